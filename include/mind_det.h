@@ -230,8 +230,9 @@ int64_t det_matmul_rmajor_f32_dev(const float *w, const float *x, float *y, int6
                                   void *stream);
 int64_t det_rows_metric_f32_dev(int64_t op, const float *w, const float *x, float *y, int64_t rows, int64_t cols,
                                 void *stream);
-/* Device form of det_fft_q16 (n >= 4096 borrows the workspace arena, whose
- * size det_fft_workspace_bytes reports). */
+/* Device form of det_fft_q16 (n >= 4096 may borrow the workspace arena, at
+ * most the size that det_fft_workspace_bytes reports; an out-of-place call
+ * needs none). */
 int64_t det_fft_q16_dev(int64_t *re, int64_t *im, const int64_t *tw, int64_t logn, int64_t n, int64_t batch,
                         void *stream);
 /* Out-of-place form: reads in_re / in_im, writes out_re / out_im (each pair

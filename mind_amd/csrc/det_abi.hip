@@ -681,11 +681,12 @@ int64_t fft_check(int64_t logn, int64_t n, int64_t batch) {
     return 0;
 }
 
-// Device-pointer FFT on stream s; the n >= 4096 path borrows the workspace
-// arena (ordered after its previous user).  Call with ds.mu NOT held.
+// Device-pointer FFT on stream s; the column passes of n >= 4096 borrow the
+// workspace arena (ordered after its previous user) unless they can write
+// the destination directly.  Call with ds.mu NOT held.
 int64_t fft_dev_run(const int64_t *sre, const int64_t *sim, int64_t *dre, int64_t *dim, const int64_t *tw, int logn,
                     int64_t batch, hipStream_t s) {
-    const size_t need = det::fft_workspace_bytes(logn, batch);
+    const size_t need = det::fft_scratch_bytes(sre, sim, dre, dim, logn, batch);
     if (need == 0) {
         DET_HIP_CHECK(det::launch_fft_q16(sre, sim, dre, dim, tw, logn, batch, nullptr, s));
         return 0;
@@ -718,7 +719,8 @@ int64_t fft_host(int64_t re, int64_t im, int64_t tw, int64_t logn, int64_t n, in
     const size_t off_im = align256(bytes), off_tw = off_im + align256(bytes);
     const size_t span = off_tw + align256(bytes_tw) + 256;
     if ((rc = ensure(&ds.io, &ds.io_bytes, span))) return rc;
-    const size_t need = det::fft_workspace_bytes((int)logn, batch);
+    const int64_t *io_re = (const int64_t *)ds.io, *io_im = (const int64_t *)((char *)ds.io + off_im);
+    const size_t need = det::fft_scratch_bytes(io_re, io_im, io_re, io_im, (int)logn, batch);
     if ((rc = ensure(&ds.ws, &ds.ws_bytes, need))) return rc;
     const bool pinned = pinned_route(ds, span);
     // a few small transforms (no workspace: one read and one write per
@@ -726,7 +728,7 @@ int64_t fft_host(int64_t re, int64_t im, int64_t tw, int64_t logn, int64_t n, in
     // the LDS kernels read each point once and write it once: in and out
     // through the pinned buffer itself on the whole pinned route (batch 64
     // of 256 points 41.5 -> 35.5 us)
-    const bool direct = pinned && need == 0;
+    const bool direct = pinned && need == 0 && logn <= 11;
     char *io = direct ? (char *)ds.pin_dev : (char *)ds.io;
     hipStream_t s = ds.stream;
     const HostIn in[3] = {{0, (const void *)re, bytes}, {off_im, (const void *)im, bytes},

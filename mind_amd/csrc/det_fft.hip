@@ -25,8 +25,9 @@
 //                      a block of transforms runs in int32 when a bound on
 //                      its inputs proves that every intermediate fits (same
 //                      integers, cheaper products), else in int64;
-//   * n >= 4096      : one global-memory pass per 4-bit window, out of place
-//                      through a workspace (fft_pass_kernel).
+//   * n >= 4096      : whole transforms in LDS up to 2^14 points
+//                      (fft_block_kernel), else passes of 6 to 10 stages over
+//                      columns of 16 points (fft_cols_kernel).
 #include "det_common.h"
 #include "det_kernels.h"
 
@@ -336,36 +337,329 @@ __global__ __launch_bounds__(256) void fft_lds_kernel(const int64_t *__restrict_
 }
 
 // ---------------------------------------------------------------- n >= 4096
-// One pass = the stages of one 4-bit window, global memory to global memory.
-// The first pass reads through the bit reversal.  Thread g: FFT g / (n/16),
-// lane-group index t = g % (n/16).
-__global__ __launch_bounds__(256) void fft_pass_kernel(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
-                                                       int64_t *__restrict__ dre, int64_t *__restrict__ dim,
-                                                       const int64_t *__restrict__ tw, int logn, int s, int b0, int b1,
-                                                       bool first, int64_t batch) {
-    const int64_t n = (int64_t)1 << logn, groups = n >> 4;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (g >= batch * groups) return;
-    const int64_t fi = g / groups;
-    const uint32_t t = (uint32_t)(g % groups);
-    const int64_t off = fi * n;
-    int64_t xr[16], xi[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pos = win_pos(t, r, s);
-        const uint32_t src = first ? bitrev(pos, logn) : pos;
-        xr[r] = sre[off + src], xi[r] = sim[off + src];
+// The stages are cut into windows of 4 position bits as above, and the
+// windows into blocks of work that live in one workgroup's LDS:
+//   * whole transforms (fft_block_kernel, n = 4096 and 8192): one workgroup
+//     per transform, one read and one write of each point;
+//   * column passes (fft_cols_kernel<NB>): a pass runs NB = 6..9 stages
+//     [s, s + NB).  A workgroup holds the 2^NB positions l << s of 16
+//     neighbouring columns, so every load and store moves runs of 16
+//     consecutive points (128 bytes) or longer, also the first pass's loads
+//     through the bit reversal: 16 neighbouring source points are 16 columns.
+//     logn / 9 passes, rounded up (10 stages would need 1024 threads of 128
+//     registers, which spill: 2 x 2^20 points 131 us in two passes, 58 in
+//     three); a pass writes the positions it reads, so every pass after the
+//     first may run in place.
+// What bounds them: a pass streams 32 bytes per point and spends about
+// 300 cycles per wave and butterfly in int64 (12 quarter-rate multiplies) or
+// 104 in int32, so the arithmetic matters as much as the stream.  A window
+// therefore runs in int32 whenever its inputs and twiddles allow it: with
+// every twiddle component within [-2^16, 2^16] a butterfly grows the largest
+// complex magnitude M to at most (1 + sqrt 2) M + 2.24 (the two floors per
+// component add an error of at most (1, 2)), so components within
+// win_bound(stages) stay below 2^31 through those stages, products included
+// (|qmul(w, x)| <= |x| + 1).  The test is repeated at each window, so only
+// the window's own growth has to be allowed for; when a test fails the block
+// starts again in int64 (nothing is stored before the last window).  Same
+// butterflies, same stage order, same integers on either path.
+// Device time per call, one global-memory pass per 4 stages whose first pass
+// gathered single 8-byte points -> this (out of place, inputs within 2^16):
+// 16 x 2^16 points 86.4 -> 25.5 us (34 MB read and written once: 6.6 us at the
+// copy rate; the two passes wait for memory, then compute, with one workgroup
+// per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
+// 61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7; inputs within
+// 2^40 (int64): 16 x 2^16 86 -> 33.7, 512 x 4096 91 -> 28.3.
+__host__ __device__ constexpr int32_t win_bound(int stages) {
+    double g = 1.0;
+    for (int i = 0; i < stages; ++i) g *= 2.4143;   // > 1 + sqrt 2
+    return (int32_t)((2147483647.0 / g - 4.0) / 1.41422);   // > sqrt 2: component -> magnitude
+}
+
+// Window P of NB bits: first bit of its 4 registers, and the stages it runs.
+template <int NB, int P>
+struct Win {
+    static constexpr int S = 4 * P < NB - 4 ? 4 * P : NB - 4, B0 = 4 * P, B1 = 4 * P + 4 < NB ? 4 * P + 4 : NB;
+};
+
+// LDS layouts.  label(): the position bits of thread t outside a window;
+// col(): its column; idx(): the 8-byte LDS element of position l, column c,
+// swizzled so that 32 consecutive lanes touch 32 different elements mod 32.
+template <int NB>
+struct BlockLay {   // a whole transform, one column
+    static constexpr int THREADS = 1 << (NB - 4), ELEMS = 1 << NB;
+    static constexpr bool FIRST = true;
+    // window 0 takes its labels bit-reversed: neighbouring threads then load
+    // neighbouring source points
+    template <int P>
+    static __device__ __forceinline__ uint32_t label(uint32_t t) { return P == 0 ? bitrev(t, NB - 4) : t; }
+    template <int P>
+    static __device__ __forceinline__ uint32_t col(uint32_t) { return 0; }
+    static __device__ __forceinline__ uint32_t idx(uint32_t l, uint32_t) {
+        // window 0 writes with lanes on the top 5 position bits, window 1 reads
+        // on bits 0..3 and 8, later windows on bits 0..4
+        uint32_t f = ((l >> 9) & 15u) ^ (((l >> 8) & 1u) << 4);
+        if (NB == 12) f ^= ((l >> 7) & 1u) << 3;
+        if (NB == 14) f ^= ((l >> 13) & 1u) << 4;
+        return l ^ f;
     }
-    run_window(xr, xi, tw, t, s, b0, b1, logn);
+};
+template <int NB, bool FIRST_>
+struct ColsLay {   // 2^NB positions of 16 columns
+    static constexpr int THREADS = 1 << NB, ELEMS = 16 << NB, NP = (NB + 3) / 4;
+    static constexpr bool FIRST = FIRST_;
+    // the first pass stores runs of consecutive positions of one column, so
+    // its last window has lanes along the positions; else lanes run along
+    // the 16 columns
+    template <int P>
+    static __device__ __forceinline__ uint32_t label(uint32_t t) {
+        return FIRST && P == NP - 1 ? t & ((1u << (NB - 4)) - 1u) : t >> 4;
+    }
+    template <int P>
+    static __device__ __forceinline__ uint32_t col(uint32_t t) {
+        return FIRST && P == NP - 1 ? t >> (NB - 4) : t & 15u;
+    }
+    static __device__ __forceinline__ uint32_t idx(uint32_t l, uint32_t c) {
+        return ((l << 4) | (c ^ (l & 15u))) ^ (l & 16u);
+    }
+};
+
+// Twiddles of window P for a thread: `low` holds the position bits below the
+// window's registers, shifted by s, and the column.  Stage bit b of the
+// transform uses table entry (position mod 2^b) << (logn - 1 - b).
+template <class L, int NB, int P, typename F>
+__device__ __forceinline__ void each_twiddle(uint32_t low, int s, int logn, F &&f) {
+    using W = Win<NB, P>;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pos = win_pos(t, r, s);
-        dre[off + pos] = xr[r], dim[off + pos] = xi[r];
+    for (int rb = 0; rb < 4; ++rb) {
+        const int bb = W::S + rb;
+        if (bb < W::B0 || bb >= W::B1) continue;
+        if (L::FIRST && bb == 0) continue;   // the peeled stage
+#pragma unroll
+        for (int q = 0; q < (1 << rb); ++q)
+            f(rb, q, (low << (logn - 1 - s - bb)) + ((uint32_t)q << (logn - 1 - rb)));
     }
 }
 
-__global__ void copy_i64_kernel(const int64_t *__restrict__ src, int64_t *__restrict__ dst, int64_t count) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256) dst[i] = src[i];
+// int32 twiddles of window P; returns whether every component is within
+// [-2^16, 2^16].
+template <class L, int NB, int P>
+__device__ __forceinline__ bool load_tw32(WinTw &w, const int64_t *__restrict__ tw, uint32_t low, int s, int logn) {
+    bool ok = true;
+    each_twiddle<L, NB, P>(low, s, logn, [&](int rb, int q, uint32_t k) {
+        const int64_t wr = tw[2 * (size_t)k], wi = tw[2 * (size_t)k + 1];
+        ok = ok && (uint64_t)(wr + TW_SMALL) <= 2 * (uint64_t)TW_SMALL &&
+             (uint64_t)(wi + TW_SMALL) <= 2 * (uint64_t)TW_SMALL;
+        w.r[(1 << rb) - 1 + q] = (int32_t)wr, w.i[(1 << rb) - 1 + q] = (int32_t)wi;
+    });
+    return ok;
+}
+
+template <class L, int NB, int P>
+__device__ __forceinline__ void run_win32(int32_t (&xr)[16], int32_t (&xi)[16], const WinTw &w) {
+    using W = Win<NB, P>;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+        const int bb = W::S + rb;
+        if (bb < W::B0 || bb >= W::B1) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if (r & (1 << rb)) continue;
+            const int slot = (1 << rb) - 1 + (r & ((1 << rb) - 1)), q = r | (1 << rb);
+            const bool peeled = L::FIRST && bb == 0;
+            butterfly(xr[r], xi[r], xr[q], xi[q], peeled ? 0 : (int64_t)w.r[slot], peeled ? 0 : (int64_t)w.i[slot],
+                      peeled);
+        }
+    }
+}
+
+template <class L, int NB, int P>
+__device__ __forceinline__ void run_win64(int64_t (&xr)[16], int64_t (&xi)[16], const int64_t *__restrict__ tw,
+                                          uint32_t low, int s, int logn) {
+    using W = Win<NB, P>;
+    // loads of its own: sharing the int32 path's would keep their 64-bit
+    // values in registers across it
+    asm volatile("" : "+s"(tw));
+    if (L::FIRST && W::B0 == 0) {   // the peeled stage
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) butterfly(xr[r], xi[r], xr[r + 1], xi[r + 1], 0, 0, true);
+    }
+    each_twiddle<L, NB, P>(low, s, logn, [&](int rb, int q, uint32_t k) {
+        const int64_t wr = tw[2 * (size_t)k], wi = tw[2 * (size_t)k + 1];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (!(r & (1 << rb)) && (r & ((1 << rb) - 1)) == q)
+                butterfly(xr[r], xi[r], xr[r | (1 << rb)], xi[r | (1 << rb)], wr, wi, false);
+    });
+}
+
+// Block-wide AND, known to the compiler as uniform.
+__device__ __forceinline__ bool block_all(bool v) { return __builtin_amdgcn_readfirstlane(__syncthreads_and(v)); }
+
+// Re-layout from window P - 1 to window P.
+template <class L, int NB, int P, typename T>
+__device__ __forceinline__ void exchange(T (&x)[16], uint32_t t, T *sm) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        sm[L::idx(win_pos(L::template label<P - 1>(t), r, Win<NB, P - 1>::S), L::template col<P - 1>(t))] = x[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        x[r] = sm[L::idx(win_pos(L::template label<P>(t), r, Win<NB, P>::S), L::template col<P>(t))];
+    __syncthreads();
+}
+
+template <class L, int NB, int P>
+__device__ __forceinline__ uint32_t low_bits(uint32_t t, int s, uint32_t c0) {
+    const uint32_t jl = L::template label<P>(t) & ((1u << Win<NB, P>::S) - 1u);
+    return L::FIRST ? jl : (jl << s) | (c0 + L::template col<P>(t));
+}
+
+// Windows P.. of the int32 path.  Where window 0's twiddles are uniform
+// (L::FIRST) w holds window P's (w_ok: all small), loaded one window ahead;
+// in later passes that would cost the second wave per SIMD (16 transforms of
+// 2^16 25.8 us instead of 27, 32 of them 41.9 instead of 38.6), so they are
+// loaded here.  Returns false when a window's test fails.
+template <class L, int NB, int P>
+__device__ __forceinline__ bool narrow_from(int32_t (&yr)[16], int32_t (&yi)[16], const int64_t *__restrict__ tw,
+                                            uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, WinTw &w, bool w_ok) {
+    if constexpr (P < (NB + 3) / 4) {
+        constexpr int32_t B = win_bound(Win<NB, P>::B1 - Win<NB, P>::B0);
+        WinTw wn;
+        bool wn_ok = true;
+        if constexpr (!L::FIRST) w_ok = load_tw32<L, NB, P>(w, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
+        else if constexpr (P + 1 < (NB + 3) / 4)
+            wn_ok = load_tw32<L, NB, P + 1>(wn, tw, low_bits<L, NB, P + 1>(t, s, c0), s, logn);
+        int32_t hi = yr[0], lo = yr[0];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            hi = max(max(hi, yr[r]), yi[r]);
+            lo = min(min(lo, yr[r]), yi[r]);
+        }
+        if (!block_all(w_ok && hi <= B && lo >= -B)) return false;
+        uint64_t z[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r] = (uint64_t)(uint32_t)yr[r] | ((uint64_t)(uint32_t)yi[r] << 32);
+        exchange<L, NB, P>(z, t, sm);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) yr[r] = (int32_t)(uint32_t)z[r], yi[r] = (int32_t)(uint32_t)(z[r] >> 32);
+        run_win32<L, NB, P>(yr, yi, w);
+        return narrow_from<L, NB, P + 1>(yr, yi, tw, t, s, c0, logn, sm, wn, wn_ok);
+    }
+    return true;
+}
+
+template <class L, int NB, int P>
+__device__ __forceinline__ void wide_from(int64_t (&xr)[16], int64_t (&xi)[16], const int64_t *__restrict__ tw,
+                                          uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm) {
+    if constexpr (P < (NB + 3) / 4) {
+        if constexpr (P > 0) {
+            exchange<L, NB, P>(xr, t, (int64_t *)sm);
+            exchange<L, NB, P>(xi, t, (int64_t *)sm);
+        }
+        run_win64<L, NB, P>(xr, xi, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
+        wide_from<L, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm);
+    }
+}
+
+// All NB stages [s, s + NB): load(r, re, im) gives window 0's points (twice
+// if need be), store(r, re, im) takes the last window's.
+template <class L, int NB, typename LD, typename ST>
+__device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_t t, int s, uint32_t c0, int logn,
+                                         uint64_t *sm, LD &&load, ST &&store) {
+    int64_t xr[16], xi[16];
+    {
+        constexpr int64_t B = win_bound(Win<NB, 0>::B1);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) load(r, xr[r], xi[r]);
+        WinTw w, w1;
+        bool ok = load_tw32<L, NB, 0>(w, tw, low_bits<L, NB, 0>(t, s, c0), s, logn);
+        bool ok1 = true;
+        if constexpr (L::FIRST) ok1 = load_tw32<L, NB, 1>(w1, tw, low_bits<L, NB, 1>(t, s, c0), s, logn);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            ok = ok && (uint64_t)(xr[r] + B) <= 2 * (uint64_t)B && (uint64_t)(xi[r] + B) <= 2 * (uint64_t)B;
+        if (block_all(ok)) {
+            int32_t yr[16], yi[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) yr[r] = (int32_t)xr[r], yi[r] = (int32_t)xi[r];
+            run_win32<L, NB, 0>(yr, yi, w);
+            if (narrow_from<L, NB, 1>(yr, yi, tw, t, s, c0, logn, sm, w1, ok1)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) store(r, (int64_t)yr[r], (int64_t)yi[r]);
+                return;
+            }
+        }
+    }
+    // nothing has been stored: the int64 path starts again from the source
+    // (keeping the loaded or the int32 values for it would hold 64 registers
+    // across the int32 path, one wave per SIMD fewer)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < 16; ++r) load(r, xr[r], xi[r]);
+    wide_from<L, NB, 0>(xr, xi, tw, t, s, c0, logn, sm);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) store(r, xr[r], xi[r]);
+}
+
+// One workgroup per transform (in place allowed: a workgroup holds its whole
+// transform before it stores).
+template <int LOGN>
+__global__ __launch_bounds__(1 << (LOGN - 4)) void fft_block_kernel(const int64_t *sre, const int64_t *sim,
+                                                                    int64_t *dre, int64_t *dim,
+                                                                    const int64_t *__restrict__ tw) {
+    using L = BlockLay<LOGN>;
+    constexpr int NP = (LOGN + 3) / 4;
+    __shared__ uint64_t sm[L::ELEMS];
+    const uint32_t t = threadIdx.x;
+    const int64_t off = (int64_t)blockIdx.x << LOGN;
+    auto load = [&](int r, int64_t &re, int64_t &im) {
+        const uint32_t src = (bitrev((uint32_t)r, 4) << (LOGN - 4)) | t;
+        re = sre[off + src], im = sim[off + src];
+    };
+    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](int r, int64_t re, int64_t im) {
+        const uint32_t pos = win_pos(L::template label<NP - 1>(t), r, Win<LOGN, NP - 1>::S);
+        dre[off + pos] = re, dim[off + pos] = im;
+    });
+}
+
+// Stages [s, s + NB) of 16 columns; grid: 2^lgb workgroups per transform.
+// The first pass (s = 0) reads through the bit reversal: its columns are the
+// low logn - NB bits of the source index (the high position bits, reversed),
+// and its source must not overlap its destination.
+template <int NB, bool FIRST>
+__global__ __launch_bounds__(1 << NB) void fft_cols_kernel(const int64_t *sre, const int64_t *sim, int64_t *dre,
+                                                           int64_t *dim, const int64_t *__restrict__ tw, int logn,
+                                                           int s, int lgb) {
+    using L = ColsLay<NB, FIRST>;
+    constexpr int NP = (NB + 3) / 4;
+    __shared__ uint64_t sm[L::ELEMS];
+    const uint32_t t = threadIdx.x, blk = blockIdx.x & ((1u << lgb) - 1u);
+    const int64_t off = (int64_t)(blockIdx.x >> lgb) << logn;
+    const uint32_t c0 = (FIRST ? blk : blk & ((1u << (s - 4)) - 1u)) << 4;
+    const uint32_t high = FIRST ? 0u : (blk >> (s - 4)) << (s + NB);
+    const uint32_t j = t >> 4, c = c0 + (t & 15u);
+    const uint32_t base = FIRST ? (bitrev(j, NB - 4) << (logn - NB)) | c : high | (j << (s + 4)) | c;
+    auto load = [&](int r, int64_t &re, int64_t &im) {
+        const uint32_t src = base + (FIRST ? bitrev((uint32_t)r, 4) << (logn - 4) : (uint32_t)r << s);
+        re = sre[off + src], im = sim[off + src];
+    };
+    run_pass<L, NB>(tw, t, s, c0, logn, sm, load, [&](int r, int64_t re, int64_t im) {
+        const uint32_t l = win_pos(L::template label<NP - 1>(t), r, Win<NB, NP - 1>::S);
+        const uint32_t cc = c0 + L::template col<NP - 1>(t);
+        const uint32_t pos = FIRST ? (bitrev(cc, logn - NB) << NB) | l : high | (l << s) | cc;
+        dre[off + pos] = re, dim[off + pos] = im;
+    });
+}
+
+template <int NB>
+static void launch_cols(const int64_t *sre, const int64_t *sim, int64_t *dre, int64_t *dim, const int64_t *tw,
+                        int logn, int s, int64_t batch, hipStream_t st) {
+    const int lgb = logn - NB - 4;
+    const dim3 grid((unsigned)(batch << lgb)), block(1u << NB);
+    if (s == 0)
+        hipLaunchKernelGGL((fft_cols_kernel<NB, true>), grid, block, 0, st, sre, sim, dre, dim, tw, logn, s, lgb);
+    else
+        hipLaunchKernelGGL((fft_cols_kernel<NB, false>), grid, block, 0, st, sre, sim, dre, dim, tw, logn, s, lgb);
 }
 
 // A few transforms (batch <= FEW_BATCH, 32 <= n <= 2048): one workgroup per
@@ -417,14 +711,45 @@ __global__ __launch_bounds__(1024) void fft_few_kernel(const int64_t *__restrict
 
 }  // namespace fft
 
+// The largest scratch any call of this size takes (a call whose first pass may
+// write its destination directly takes none: fft_scratch_bytes).
 size_t fft_workspace_bytes(int logn, int64_t batch) {
     if (logn <= 11) return 0;
     return 2 * (size_t)batch * ((size_t)1 << logn) * sizeof(int64_t);
 }
 
+namespace fft {
+static bool overlap(const int64_t *a, const int64_t *b, int64_t count) { return a < b + count && b < a + count; }
+
+// Whole transforms per workgroup: 4096 points always (1 transform 9.5 us
+// against 10.9 in two passes, 64 10.2 against 13.2), 8192 once there are 128
+// of them (21.8 us against 24.5; 64 21.5 against 16.1).  In place (or
+// disjoint) only: a workgroup reads its own transform alone.
+static bool whole(const int64_t *sre, const int64_t *sim, const int64_t *dre, const int64_t *dim, int logn,
+                  int64_t batch) {
+    if (logn > 13 || batch < (logn == 12 ? 1 : 128)) return false;
+    const int64_t cnt = batch << logn;
+    return !overlap(sre, dim, cnt) && !overlap(sim, dre, cnt) && (sre == dre || !overlap(sre, dre, cnt)) &&
+           (sim == dim || !overlap(sim, dim, cnt));
+}
+}  // namespace fft
+
+// Scratch a call takes: the first column pass permutes points across
+// workgroups, so it goes through scratch when a source range overlaps a
+// destination range.
+size_t fft_scratch_bytes(const int64_t *sre, const int64_t *sim, const int64_t *dre, const int64_t *dim, int logn,
+                         int64_t batch) {
+    using namespace fft;
+    if (logn <= 11 || whole(sre, sim, dre, dim, logn, batch)) return 0;
+    const int64_t cnt = batch << logn;
+    const bool any = overlap(sre, dre, cnt) || overlap(sre, dim, cnt) || overlap(sim, dre, cnt) ||
+                     overlap(sim, dim, cnt);
+    return any ? fft_workspace_bytes(logn, batch) : 0;
+}
+
 // batch transforms of n = 2^logn points: transform f read from sre / sim
 // + f n and written to dre / dim + f n (the same pointers for in place).
-// logn in [0, 30]; ws: fft_workspace_bytes(logn, batch) bytes.
+// logn in [0, 30]; ws: fft_scratch_bytes() bytes.
 hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, int64_t *dim, const int64_t *tw,
                           int logn, int64_t batch, void *ws, hipStream_t s) {
     using namespace fft;
@@ -456,28 +781,28 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
     LDS(5) LDS(6) LDS(7) LDS(8) LDS(9) LDS(10) LDS(11)
 #undef LDS
     default: {
-        if (!ws) return hipErrorInvalidValue;
-        int64_t *wre = (int64_t *)ws, *wim = wre + batch * n;
-        const int np = (logn + 3) / 4;
-        const int64_t threads = batch * (n >> 4);
-        const dim3 grid((unsigned)((threads + 255) / 256));
-        // pass 0 reads the source through the bit reversal into the
-        // workspace; later passes alternate dst and workspace; an odd pass
-        // count ends in the workspace and is copied to dst
-        const int64_t *src_re = sre, *src_im = sim;
-        for (int p = 0; p < np; ++p) {
-            const int sw = 4 * p < logn - 4 ? 4 * p : logn - 4;
-            const int b1 = 4 * p + 4 < logn ? 4 * p + 4 : logn;
-            int64_t *to_re = (p % 2 == 0) ? wre : dre, *to_im = (p % 2 == 0) ? wim : dim;
-            hipLaunchKernelGGL(fft_pass_kernel, grid, dim3(256), 0, s, src_re, src_im, to_re, to_im, tw, logn, sw,
-                               4 * p, b1, p == 0, batch);
-            src_re = to_re, src_im = to_im;
+        if (whole(sre, sim, dre, dim, logn, batch)) {
+            const dim3 grid((unsigned)batch), block(1u << (logn - 4));
+            if (logn == 12) hipLaunchKernelGGL(fft_block_kernel<12>, grid, block, 0, s, sre, sim, dre, dim, tw);
+            else hipLaunchKernelGGL(fft_block_kernel<13>, grid, block, 0, s, sre, sim, dre, dim, tw);
+            break;
         }
-        if (src_re == wre) {
-            const int64_t cnt = batch * n;
-            const unsigned gb = (unsigned)((cnt + 255) / 256 < cap ? (cnt + 255) / 256 : cap);
-            hipLaunchKernelGGL(copy_i64_kernel, dim3(gb), dim3(256), 0, s, wre, dre, cnt);
-            hipLaunchKernelGGL(copy_i64_kernel, dim3(gb), dim3(256), 0, s, wim, dim, cnt);
+        const bool scratch = fft_scratch_bytes(sre, sim, dre, dim, logn, batch) != 0;
+        if (scratch && !ws) return hipErrorInvalidValue;
+        const int np = (logn + 8) / 9;
+        const int64_t *from_re = sre, *from_im = sim;
+        for (int p = 0, b = 0; p < np; ++p) {
+            const int nb = (logn - b + np - p - 1) / (np - p);   // the rest, split evenly
+            int64_t *to_re = scratch && p == 0 ? (int64_t *)ws : dre;
+            int64_t *to_im = scratch && p == 0 ? (int64_t *)ws + batch * n : dim;
+            switch (nb) {
+            case 6: launch_cols<6>(from_re, from_im, to_re, to_im, tw, logn, b, batch, s); break;
+            case 7: launch_cols<7>(from_re, from_im, to_re, to_im, tw, logn, b, batch, s); break;
+            case 8: launch_cols<8>(from_re, from_im, to_re, to_im, tw, logn, b, batch, s); break;
+            default: launch_cols<9>(from_re, from_im, to_re, to_im, tw, logn, b, batch, s); break;
+            }
+            b += nb;
+            from_re = to_re, from_im = to_im;
         }
         break;
     }

@@ -529,6 +529,49 @@ def test_fft_out_of_place_and_path_choice():
         b.free()
 
 
+# Transforms of 4096 points and more: whole transforms per workgroup (4096
+# points; 8192 from a batch of 128) or column passes of 6 to 9 stages (every
+# width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
+# scratch) and out of place.  Amplitudes: Q16; around the bound up to which a
+# four-stage window runs in int32 (about 44.7 million: the window after it then fails
+# its test and the block starts again in int64); +-2^40.
+FFT_LONG = [(12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
+
+
+@pytest.mark.parametrize("logn,batch", FFT_LONG, ids=[f"n{1 << l}_b{b}" for l, b in FFT_LONG])
+def test_fft_long_passes(logn, batch):
+    n, s = 1 << logn, M.Stream()
+    rng = np.random.default_rng(logn * 977 + batch)
+    std = O.fft_twiddles(n)
+    big = std.copy()
+    big[rng.integers(2, n)] = 70000        # one component above 2^16: only its users leave int32
+    sel = sorted({0, batch // 2, batch - 1})
+    g = 2.4143 ** 4
+    bound = int((2147483647.0 / g - 4.0) / 1.41422)
+    for amp, tw in ((1 << 16, std), (1 << 16, big), (bound - 1, std), (bound + 2, std), (1 << 40, std)):
+        x = rng.integers(-amp, amp, (2, batch, n), endpoint=True)
+        if batch > 2:
+            x[:, 1] >>= 12                  # a batch that mixes both paths
+        re, im = np.ascontiguousarray(x[0]), np.ascontiguousarray(x[1])
+        want = _fft_oracle_batch(re[sel], im[sel], tw, logn)
+        sre, sim, dtw = M.DeviceBuffer.from_array(re), M.DeviceBuffer.from_array(im), M.DeviceBuffer.from_array(tw)
+        dre, dim_ = M.DeviceBuffer(re.nbytes), M.DeviceBuffer(im.nbytes)
+        dre.fill(0x3C), dim_.fill(0x3C)
+        note(f"fft long n={n} batch={batch} amp={amp}")
+        M.check(M.lib().det_fft_q16_oop_dev(sre.ptr, sim.ptr, dre.ptr, dim_.ptr, dtw.ptr, logn, n, batch, s.ptr))
+        s.sync()
+        assert np.array_equal(dre.to_array(np.int64, re.shape)[sel], want[0])
+        assert np.array_equal(dim_.to_array(np.int64, re.shape)[sel], want[1])
+        assert np.array_equal(sre.to_array(np.int64, re.shape), re)
+        M.check(M.lib().det_fft_q16_dev(sre.ptr, sim.ptr, dtw.ptr, logn, n, batch, s.ptr))
+        s.sync()
+        assert np.array_equal(sre.to_array(np.int64, re.shape)[sel], want[0])
+        assert np.array_equal(sim.to_array(np.int64, re.shape)[sel], want[1])
+        for b in (sre, sim, dre, dim_, dtw):
+            b.free()
+    s.destroy()
+
+
 def test_fft_argument_conventions():
     L = M.lib()
     z = np.zeros(16, np.int64)
