@@ -19,15 +19,15 @@
 // bits, lane index t = the other bits) and runs the stages of that window in
 // registers:
 //   * n <= 16        : one FFT per thread (fft_small_kernel);
-//   * 32 <= n <= 2048: n / 16 lanes per FFT, passes separated by an LDS
-//                      transpose, bit reversal folded into the first load,
-//                      one HBM read and one write per point (fft_lds_kernel);
-//                      a block of transforms runs in int32 when a bound on
-//                      its inputs proves that every intermediate fits (same
-//                      integers, cheaper products), else in int64;
-//   * n >= 4096      : whole transforms in LDS up to 2^14 points
-//                      (fft_block_kernel), else passes of 6 to 10 stages over
-//                      columns of 16 points (fft_cols_kernel).
+//   * 32 <= n <= 2048: whole transforms in one workgroup, n / 16 lanes each,
+//                      windows separated by an LDS transpose, one HBM read
+//                      and one write per point (fft_rows_kernel up to 512
+//                      points, fft_block_kernel above; fft_few_kernel for a
+//                      few transforms);
+//   * n >= 4096      : the same up to 8192 points, else passes of 6 to 9
+//                      stages over columns of 16 points (fft_cols_kernel).
+// A window runs in int32 when a bound on its inputs proves that every
+// intermediate fits (same integers, cheaper products), else in int64.
 #include "det_common.h"
 #include "det_kernels.h"
 
@@ -64,14 +64,19 @@ __device__ __forceinline__ void butterfly(V &ar, V &ai, V &br, V &bi, int64_t wr
     br = vsub(ur, tr), bi = vsub(ui, ti);
 }
 
-// Largest input magnitude for which a 2^logn-point transform stays in int32
-// when every twiddle component is within [-2^16, 2^16]: |qmul(w, x)| <= |x|,
-// so a span-2 stage at most doubles the largest magnitude and each later
-// stage at most triples it (|a +- (qmul - qmul)| <= 3 max).
-__host__ __device__ constexpr int64_t i32_input_bound(int logn) {
-    int64_t g = logn >= 1 ? 2 : 1;
-    for (int i = 1; i < logn; ++i) g *= 3;
-    return 2147483647LL / g;
+// Largest input component for which `stages` stages (the first of them peeled
+// if `peeled`) stay in int32 when every twiddle component is within
+// [-2^16, 2^16].  A twiddle then has complex magnitude at most sqrt 2, and the
+// floors of the two products of a component add an error of at most (1, 2), so
+// a butterfly takes the largest magnitude M to at most
+// (1 + sqrt 2) M + 2.24 (a peeled one to 2 M): components stay below 2^31, and
+// so do the products, |qmul(w, x)| <= |x| + 1.  A component-wise bound (each
+// stage triples the largest component) would send n >= 1024 with Q16 inputs in
+// [-1, 1) to int64.
+__host__ __device__ constexpr int32_t i32_bound(int stages, bool peeled) {
+    double g = peeled ? 2.0 : 1.0;
+    for (int i = peeled ? 1 : 0; i < stages; ++i) g *= 2.4143;   // > 1 + sqrt 2
+    return (int32_t)((2147483647.0 / g - 4.0) / 1.41422);        // > sqrt 2: component -> magnitude
 }
 constexpr int64_t TW_SMALL = 65536;
 
@@ -82,98 +87,14 @@ __device__ __forceinline__ uint32_t win_pos(uint32_t t, int r, int s) {
     return ((t >> s) << (s + 4)) | ((uint32_t)r << s) | (t & ((1u << s) - 1u));
 }
 
-// Stage b = s + RB of a window at s: butterflies between registers r and
-// r | 2^RB (register indices are compile-time, so the points stay in VGPRs).
-template <int RB, typename V>
-__device__ __forceinline__ void window_stage(V (&xr)[16], V (&xi)[16], const int64_t *__restrict__ tw,
-                                             uint32_t t, int s, int logn) {
-    const int b = s + RB;
-    const uint32_t half_mask = (1u << b) - 1u;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        if (r & (1 << RB)) continue;
-        constexpr int bit = 1 << RB;
-        int64_t wr = 0, wi = 0;
-        if (b > 0) {
-            const uint32_t k = (win_pos(t, r, s) & half_mask) << (logn - 1 - b);
-            wr = tw[2 * k], wi = tw[2 * k + 1];
-        }
-        butterfly(xr[r], xi[r], xr[r | bit], xi[r | bit], wr, wi, b == 0);
-    }
-}
-
-// Stages [b0, b1) of a window at s (b0 >= s, b1 <= s + 4), in order.
-template <typename V>
-__device__ __forceinline__ void run_window(V (&xr)[16], V (&xi)[16], const int64_t *__restrict__ tw,
-                                           uint32_t t, int s, int b0, int b1, int logn) {
-    if (b0 <= s && s < b1) window_stage<0>(xr, xi, tw, t, s, logn);
-    if (b0 <= s + 1 && s + 1 < b1) window_stage<1>(xr, xi, tw, t, s, logn);
-    if (b0 <= s + 2 && s + 2 < b1) window_stage<2>(xr, xi, tw, t, s, logn);
-    if (b0 <= s + 3 && s + 3 < b1) window_stage<3>(xr, xi, tw, t, s, logn);
-}
-
-// ---- int32 path: twiddles preloaded as int32 (valid when every component
-// is within [-2^16, 2^16]).  Slot (2^rb - 1) + j of a window's table holds
+// A window's twiddles on the int32 path (valid when every component is
+// within [-2^16, 2^16]).  Slot (2^rb - 1) + j of a window's table holds
 // the twiddle of stage s + rb for butterflies whose register index has low
 // bits j (the position bits below the stage bit are those low bits and the
 // lane's own bits, so 1 + 2 + 4 + 8 slots cover a window).
 struct WinTw {
     int32_t r[15], i[15];
 };
-
-template <int S, int B0, int B1, int LOGN>
-__device__ __forceinline__ void load_win_tw(WinTw &w, const int64_t *__restrict__ tw, uint32_t t) {
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-        const int b = S + rb;
-        if (b < B0 || b >= B1 || b == 0) continue;
-#pragma unroll
-        for (int j = 0; j < (1 << rb); ++j) {
-            const uint32_t k = (win_pos(t, j, S) & ((1u << b) - 1u)) << (LOGN - 1 - b);
-            int32_t wr = (int32_t)tw[2 * k], wi = (int32_t)tw[2 * k + 1];
-            if (S == 0) {   // window 0: the same twiddles in every lane
-                wr = __builtin_amdgcn_readfirstlane(wr);
-                wi = __builtin_amdgcn_readfirstlane(wi);
-            }
-            w.r[(1 << rb) - 1 + j] = wr, w.i[(1 << rb) - 1 + j] = wi;
-        }
-    }
-}
-
-template <int S, int B0, int B1>
-__device__ __forceinline__ void window32(int32_t (&xr)[16], int32_t (&xi)[16], const WinTw &w) {
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-        const int b = S + rb;
-        if (b < B0 || b >= B1) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            if (r & (1 << rb)) continue;
-            const int slot = (1 << rb) - 1 + (r & ((1 << rb) - 1));
-            const int q = r | (1 << rb);
-            butterfly(xr[r], xi[r], xr[q], xi[q], (int64_t)w.r[slot], (int64_t)w.i[slot], b == 0);
-        }
-    }
-}
-
-// Re-layout from window SP to window S through LDS, (re, im) as one 8-byte
-// element at index pos + pos / 16.
-template <int SP, int S>
-__device__ __forceinline__ void transpose32(int32_t (&xr)[16], int32_t (&xi)[16], uint32_t t, uint64_t *smf) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pos = win_pos(t, r, SP);
-        smf[pos + (pos >> 4)] = (uint64_t)(uint32_t)xr[r] | ((uint64_t)(uint32_t)xi[r] << 32);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pos = win_pos(t, r, S);
-        const uint64_t v = smf[pos + (pos >> 4)];
-        xr[r] = (int32_t)(uint32_t)v, xi[r] = (int32_t)(uint32_t)(v >> 32);
-    }
-    __syncthreads();
-}
 
 // ---------------------------------------------------------------- n <= 16
 // One thread per FFT; registers indexed by position.
@@ -208,139 +129,13 @@ __global__ __launch_bounds__(256) void fft_small_kernel(const int64_t *__restric
     for (int p = 0; p < N; ++p) dre[f * N + p] = xr[p], dim[f * N + p] = xi[p];
 }
 
-// ---------------------------------------------------------------- 32 <= n <= 2048
-// L = n / 16 lanes per FFT, 256 / L FFTs per 256-thread block, a block-
-// uniform grid-stride loop over the batch.  Reads src, writes dst (equal for
-// in place: a lane group holds its whole transform before storing).  LDS
-// holds one component of every FFT of the block at a time, index
-// pos + pos / 16 (one pad element per 16, so the 16 lanes of a window hit
-// distinct banks).  Per block of transforms the path is chosen once, block-
-// uniformly (the LDS transposes need the whole block): int32 when the table
-// is small and every loaded value is within i32_input_bound, else int64.
-template <int LOGN, typename V>
-__device__ __forceinline__ void lds_transform(V (&xr)[16], V (&xi)[16], const int64_t *__restrict__ tw, uint32_t t,
-                                              V *smf) {
-    constexpr int N = 1 << LOGN, NP = (LOGN + 3) / 4;
-    run_window(xr, xi, tw, t, 0, 0, 4, LOGN);
-#pragma unroll
-    for (int p = 1; p < NP; ++p) {
-        const int sp = 4 * (p - 1) < LOGN - 4 ? 4 * (p - 1) : LOGN - 4;   // previous window
-        const int s = 4 * p < LOGN - 4 ? 4 * p : LOGN - 4;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            V(&x)[16] = c ? xi : xr;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t pos = win_pos(t, r, sp);
-                smf[pos + (pos >> 4)] = x[r];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t pos = win_pos(t, r, s);
-                x[r] = smf[pos + (pos >> 4)];
-            }
-            __syncthreads();
-        }
-        run_window(xr, xi, tw, t, s, 4 * p, 4 * p + 4 < LOGN ? 4 * p + 4 : LOGN, LOGN);
-    }
-    (void)N;
-}
-
-// A block handles FPB transforms at a time ("group" f0 .. f0 + FPB - 1);
-// lane t of slot f loads window 0 of transform f0 + f.
-template <int LOGN>
-__device__ __forceinline__ bool load_group(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
-                                           int64_t fi, bool live, uint32_t t, int64_t (&xr)[16], int64_t (&xi)[16]) {
-    constexpr int N = 1 << LOGN;
-    constexpr int64_t BOUND = i32_input_bound(LOGN);
-    const int64_t off = (live ? fi : 0) * N;
-    // window 0 (s = 0): position 16 t + r holds x[bitrev(16 t + r)]
-    const uint32_t tb = bitrev(t, LOGN - 4);
-    bool fits = true;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t src = (bitrev((uint32_t)r, 4) << (LOGN - 4)) | tb;
-        xr[r] = live ? __builtin_nontemporal_load(sre + off + src) : 0;   // each point is read once
-        xi[r] = live ? __builtin_nontemporal_load(sim + off + src) : 0;
-        fits = fits && xr[r] >= -BOUND && xr[r] <= BOUND && xi[r] >= -BOUND && xi[r] <= BOUND;
-    }
-    return fits;
-}
-
-template <int LOGN, typename V>
-__device__ __forceinline__ void store_group(int64_t *__restrict__ dre, int64_t *__restrict__ dim, int64_t fi,
-                                            uint32_t t, const V (&xr)[16], const V (&xi)[16]) {
-    constexpr int N = 1 << LOGN, NP = (LOGN + 3) / 4;
-    constexpr int S_LAST = 4 * (NP - 1) < LOGN - 4 ? 4 * (NP - 1) : LOGN - 4;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pos = win_pos(t, r, S_LAST);
-        __builtin_nontemporal_store((int64_t)xr[r], dre + fi * N + pos);   // streamed: read by no one here
-        __builtin_nontemporal_store((int64_t)xi[r], dim + fi * N + pos);
-    }
-}
-
-// A block of transforms whose inputs are all within i32_input_bound (and a
-// table within [-2^16, 2^16]) runs in int32; any other block runs the int64
-// transform on the values it has already loaded (the choice is block-uniform,
-// so every thread takes the same path through the LDS transposes).
-template <int LOGN>
-__global__ __launch_bounds__(256) void fft_lds_kernel(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
-                                                      int64_t *__restrict__ dre, int64_t *__restrict__ dim,
-                                                      const int64_t *__restrict__ tw, int64_t batch) {
-    constexpr int N = 1 << LOGN, L = N / 16, FPB = 256 / L, NP = (LOGN + 3) / 4;
-    constexpr int STRIDE = N + N / 16;
-    constexpr int S1 = 4 < LOGN - 4 ? 4 : LOGN - 4, S2 = 8 < LOGN - 4 ? 8 : LOGN - 4;
-    static_assert(LOGN >= 5 && LOGN <= 11, "LDS FFT size");
-    __shared__ uint64_t sm[FPB * STRIDE];
-    const int f = threadIdx.x / L;
-    const uint32_t t = threadIdx.x % L;
-    // every twiddle component within [-2^16, 2^16] (the standard table is)
-    bool small = true;
-    for (int i = threadIdx.x; i < N; i += 256) {
-        const int64_t w = tw[i];
-        small = small && w >= -TW_SMALL && w <= TW_SMALL;
-    }
-    const bool tw_small = __syncthreads_and(small);
-    WinTw w0, w1, w2;
-    if (tw_small) {
-        load_win_tw<0, 0, 4, LOGN>(w0, tw, t);
-        if constexpr (NP > 1) load_win_tw<S1, 4, (8 < LOGN ? 8 : LOGN), LOGN>(w1, tw, t);
-        if constexpr (NP > 2) load_win_tw<S2, 8, LOGN, LOGN>(w2, tw, t);
-    }
-    uint64_t *smf = sm + f * STRIDE;
-    for (int64_t f0 = (int64_t)blockIdx.x * FPB; f0 < batch; f0 += (int64_t)gridDim.x * FPB) {
-        const int64_t fi = f0 + f;
-        const bool live = fi < batch;
-        int64_t xr[16], xi[16];
-        const bool fits = load_group<LOGN>(sre, sim, fi, live, t, xr, xi);
-        if (!__syncthreads_and(fits && tw_small)) {
-            lds_transform<LOGN>(xr, xi, tw, t, (int64_t *)smf);
-            if (live) store_group<LOGN>(dre, dim, fi, t, xr, xi);
-            continue;
-        }
-        int32_t yr[16], yi[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) yr[r] = (int32_t)xr[r], yi[r] = (int32_t)xi[r];
-        window32<0, 0, 4>(yr, yi, w0);
-        if constexpr (NP > 1) {
-            transpose32<0, S1>(yr, yi, t, smf);
-            window32<S1, 4, (8 < LOGN ? 8 : LOGN)>(yr, yi, w1);
-        }
-        if constexpr (NP > 2) {
-            transpose32<S1, S2>(yr, yi, t, smf);
-            window32<S2, 8, LOGN>(yr, yi, w2);
-        }
-        if (live) store_group<LOGN>(dre, dim, fi, t, yr, yi);
-    }
-}
-
-// ---------------------------------------------------------------- n >= 4096
+// ---------------------------------------------------------------- n >= 32
 // The stages are cut into windows of 4 position bits as above, and the
-// windows into blocks of work that live in one workgroup's LDS:
-//   * whole transforms (fft_block_kernel, n = 4096 and 8192): one workgroup
-//     per transform, one read and one write of each point;
+// windows into pieces of work that live in one workgroup's LDS:
+//   * short transforms (fft_rows_kernel, n <= 512): 4096 consecutive points
+//     per workgroup;
+//   * whole transforms (fft_block_kernel, n = 1024 .. 8192): one workgroup per
+//     transform;
 //   * column passes (fft_cols_kernel<NB>): a pass runs NB = 6..9 stages
 //     [s, s + NB).  A workgroup holds the 2^NB positions l << s of 16
 //     neighbouring columns, so every load and store moves runs of 16
@@ -353,28 +148,25 @@ __global__ __launch_bounds__(256) void fft_lds_kernel(const int64_t *__restrict_
 // What bounds them: a pass streams 32 bytes per point and spends about
 // 300 cycles per wave and butterfly in int64 (12 quarter-rate multiplies) or
 // 104 in int32, so the arithmetic matters as much as the stream.  A window
-// therefore runs in int32 whenever its inputs and twiddles allow it: with
-// every twiddle component within [-2^16, 2^16] a butterfly grows the largest
-// complex magnitude M to at most (1 + sqrt 2) M + 2.24 (the two floors per
-// component add an error of at most (1, 2)), so components within
-// win_bound(stages) stay below 2^31 through those stages, products included
-// (|qmul(w, x)| <= |x| + 1).  The test is repeated at each window, so only
-// the window's own growth has to be allowed for; when a test fails the block
-// starts again in int64 (nothing is stored before the last window).  Same
-// butterflies, same stage order, same integers on either path.
-// Device time per call, one global-memory pass per 4 stages whose first pass
-// gathered single 8-byte points -> this (out of place, inputs within 2^16):
-// 16 x 2^16 points 86.4 -> 25.5 us (34 MB read and written once: 6.6 us at the
-// copy rate; the two passes wait for memory, then compute, with one workgroup
-// per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
-// 61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7; inputs within
-// 2^40 (int64): 16 x 2^16 86 -> 33.7, 512 x 4096 91 -> 28.3.
-__host__ __device__ constexpr int32_t win_bound(int stages) {
-    double g = 1.0;
-    for (int i = 0; i < stages; ++i) g *= 2.4143;   // > 1 + sqrt 2
-    return (int32_t)((2147483647.0 / g - 4.0) / 1.41422);   // > sqrt 2: component -> magnitude
-}
-
+// therefore runs in int32 whenever its inputs and twiddles allow it
+// (i32_bound).  The test is repeated at each window, so only the window's own
+// growth has to be allowed for; when a test fails the block starts again in
+// int64 (nothing is stored before the last window).  Same butterflies, same
+// stage order, same integers on either path.
+// Device time per call, out of place, inputs within 2^16 (before: windows of
+// the short transforms in one kernel with an all-or-nothing int32 test that
+// left n >= 1024 in int64; one global-memory pass per 4 stages beyond, whose
+// first pass gathered single 8-byte points):
+//   65536 x 256 points 102.7 -> 95 us (5.6 TB/s; a large copy reaches 5.2),
+//   32768 x 512 150 -> 97, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 116,
+//   100000 x 64 88 -> 41-45, 100000 x 128 104 -> 76, 300000 x 32 355 -> 58-61;
+//   16 x 2^16 points 86.1 -> 25.5 (34 MB read and written once: 6.6 us at the
+//   copy rate; the two passes wait for memory, then compute, with one workgroup
+//   per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
+//   61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7.
+// Inputs within 2^40 (int64): 65536 x 256 114 -> 115, 32768 x 512 192 -> 133,
+//   13594 x 1024 231 -> 136, 8192 x 2048 302 -> 174, 100000 x 64 83 -> 58,
+//   16 x 2^16 86 -> 33.7.
 // Window P of NB bits: first bit of its 4 registers, and the stages it runs.
 template <int NB, int P>
 struct Win {
@@ -387,7 +179,8 @@ struct Win {
 template <int NB>
 struct BlockLay {   // a whole transform, one column
     static constexpr int THREADS = 1 << (NB - 4), ELEMS = 1 << NB;
-    static constexpr bool FIRST = true;
+    static constexpr bool FIRST = true, STAGED = false, KEEP = false;
+    using Wide = BlockLay;
     // window 0 takes its labels bit-reversed: neighbouring threads then load
     // neighbouring source points
     template <int P>
@@ -398,15 +191,46 @@ struct BlockLay {   // a whole transform, one column
         // window 0 writes with lanes on the top 5 position bits, window 1 reads
         // on bits 0..3 and 8, later windows on bits 0..4
         uint32_t f = ((l >> 9) & 15u) ^ (((l >> 8) & 1u) << 4);
+        if (NB == 10) f ^= ((l >> 5) & 7u) << 1;
+        if (NB == 11) f ^= ((l >> 6) & 3u) << 2;
         if (NB == 12) f ^= ((l >> 7) & 1u) << 3;
-        if (NB == 14) f ^= ((l >> 13) & 1u) << 4;
         return l ^ f;
+    }
+};
+template <int NB, bool STAGED_>
+struct RowsLay {   // 4096 consecutive points: 2^(12 - NB) whole short transforms
+    static constexpr int THREADS = 256, ELEMS = 4096;
+    static constexpr bool FIRST = true;
+    // STAGED: loads and stores are linear and go through LDS (below 256 points
+    // a window's lanes cover less than a 128-byte line of each transform).
+    // The int64 path, 16 bytes a point, is staged below 128 points only.
+    static constexpr bool STAGED = STAGED_, KEEP = !STAGED;
+    using Wide = RowsLay<NB, STAGED_ && (NB < 7)>;
+    template <int P>
+    static __device__ __forceinline__ uint32_t label(uint32_t t) {
+        const uint32_t j = t & ((1u << (NB - 4)) - 1u);
+        return P == 0 && !STAGED ? bitrev(j, NB - 4) : j;
+    }
+    template <int P>
+    static __device__ __forceinline__ uint32_t col(uint32_t t) { return t >> (NB - 4); }
+    static __device__ __forceinline__ uint32_t idx(uint32_t l, uint32_t c) {
+        // 32 lanes cover, in turn: the top 5 position bits (linear loads), the
+        // label bits 4.. and columns (window 0), the label's low bits and
+        // columns (last window), the low 5 position bits (linear stores)
+        uint32_t f = 0;
+        if (NB == 5) f = (c & 15u) ^ ((c & 1u) << 4);
+        if (NB == 6) f = ((l >> 5) & 1u) ^ ((c & 3u) << 2) ^ (((c >> 2) & 1u) * 0x12u);
+        if (NB == 7) f = ((l >> 5) & 3u) ^ ((c & 3u) << 2) ^ ((c & 1u) << 4);
+        if (NB == 8) f = ((l >> 5) & 7u) ^ ((c & 1u) * 0x18u);
+        if (NB == 9) f = ((l >> 5) & 15u) ^ (((l >> 8) & 1u) << 4);
+        return ((c << NB) | l) ^ f;
     }
 };
 template <int NB, bool FIRST_>
 struct ColsLay {   // 2^NB positions of 16 columns
     static constexpr int THREADS = 1 << NB, ELEMS = 16 << NB, NP = (NB + 3) / 4;
-    static constexpr bool FIRST = FIRST_;
+    static constexpr bool FIRST = FIRST_, STAGED = false, KEEP = false;
+    using Wide = ColsLay;
     // the first pass stores runs of consecutive positions of one column, so
     // its last window has lanes along the positions; else lanes run along
     // the 16 columns
@@ -495,17 +319,38 @@ __device__ __forceinline__ void run_win64(int64_t (&xr)[16], int64_t (&xi)[16], 
 // Block-wide AND, known to the compiler as uniform.
 __device__ __forceinline__ bool block_all(bool v) { return __builtin_amdgcn_readfirstlane(__syncthreads_and(v)); }
 
+// LDS element of register r of thread t in window P; P = -1 and NP: the
+// linear order of staged loads (element r * THREADS + t of the sources) and
+// stores.
+template <class L, int NB, int P>
+__device__ __forceinline__ uint32_t elem(uint32_t t, int r) {
+    if constexpr (P < 0 || P == (NB + 3) / 4) {
+        const uint32_t i = (uint32_t)r * L::THREADS + t, p = i & ((1u << NB) - 1u);
+        return L::idx(P < 0 ? bitrev(p, NB) : p, i >> NB);
+    } else {
+        return L::idx(win_pos(L::template label<P>(t), r, Win<NB, P>::S), L::template col<P>(t));
+    }
+}
+
 // Re-layout from window P - 1 to window P.
 template <class L, int NB, int P, typename T>
 __device__ __forceinline__ void exchange(T (&x)[16], uint32_t t, T *sm) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        sm[L::idx(win_pos(L::template label<P - 1>(t), r, Win<NB, P - 1>::S), L::template col<P - 1>(t))] = x[r];
+    for (int r = 0; r < 16; ++r) sm[elem<L, NB, P - 1>(t, r)] = x[r];
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        x[r] = sm[L::idx(win_pos(L::template label<P>(t), r, Win<NB, P>::S), L::template col<P>(t))];
+    for (int r = 0; r < 16; ++r) x[r] = sm[elem<L, NB, P>(t, r)];
     __syncthreads();
+}
+
+template <class L, int NB, int P>
+__device__ __forceinline__ void exchange32(int32_t (&yr)[16], int32_t (&yi)[16], uint32_t t, uint64_t *sm) {
+    uint64_t z[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z[r] = (uint64_t)(uint32_t)yr[r] | ((uint64_t)(uint32_t)yi[r] << 32);
+    exchange<L, NB, P>(z, t, sm);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) yr[r] = (int32_t)(uint32_t)z[r], yi[r] = (int32_t)(uint32_t)(z[r] >> 32);
 }
 
 template <class L, int NB, int P>
@@ -523,7 +368,7 @@ template <class L, int NB, int P>
 __device__ __forceinline__ bool narrow_from(int32_t (&yr)[16], int32_t (&yi)[16], const int64_t *__restrict__ tw,
                                             uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, WinTw &w, bool w_ok) {
     if constexpr (P < (NB + 3) / 4) {
-        constexpr int32_t B = win_bound(Win<NB, P>::B1 - Win<NB, P>::B0);
+        constexpr int32_t B = i32_bound(Win<NB, P>::B1 - Win<NB, P>::B0, false);
         WinTw wn;
         bool wn_ok = true;
         if constexpr (!L::FIRST) w_ok = load_tw32<L, NB, P>(w, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
@@ -536,12 +381,7 @@ __device__ __forceinline__ bool narrow_from(int32_t (&yr)[16], int32_t (&yi)[16]
             lo = min(min(lo, yr[r]), yi[r]);
         }
         if (!block_all(w_ok && hi <= B && lo >= -B)) return false;
-        uint64_t z[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) z[r] = (uint64_t)(uint32_t)yr[r] | ((uint64_t)(uint32_t)yi[r] << 32);
-        exchange<L, NB, P>(z, t, sm);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) yr[r] = (int32_t)(uint32_t)z[r], yi[r] = (int32_t)(uint32_t)(z[r] >> 32);
+        exchange32<L, NB, P>(yr, yi, t, sm);
         run_win32<L, NB, P>(yr, yi, w);
         return narrow_from<L, NB, P + 1>(yr, yi, tw, t, s, c0, logn, sm, wn, wn_ok);
     }
@@ -552,25 +392,30 @@ template <class L, int NB, int P>
 __device__ __forceinline__ void wide_from(int64_t (&xr)[16], int64_t (&xi)[16], const int64_t *__restrict__ tw,
                                           uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm) {
     if constexpr (P < (NB + 3) / 4) {
-        if constexpr (P > 0) {
+        if constexpr (P > 0 || L::STAGED) {
             exchange<L, NB, P>(xr, t, (int64_t *)sm);
             exchange<L, NB, P>(xi, t, (int64_t *)sm);
         }
         run_win64<L, NB, P>(xr, xi, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
         wide_from<L, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm);
+    } else if constexpr (L::STAGED) {
+        exchange<L, NB, P>(xr, t, (int64_t *)sm);
+        exchange<L, NB, P>(xi, t, (int64_t *)sm);
     }
 }
 
-// All NB stages [s, s + NB): load(r, re, im) gives window 0's points (twice
-// if need be), store(r, re, im) takes the last window's.
+// All NB stages [s, s + NB): load(layout, r, re, im) gives window 0's points
+// (twice if need be), store(layout, r, re, im) takes the last window's (linear
+// order on both sides where staged).
 template <class L, int NB, typename LD, typename ST>
 __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_t t, int s, uint32_t c0, int logn,
                                          uint64_t *sm, LD &&load, ST &&store) {
     int64_t xr[16], xi[16];
+    bool narrow = false;
     {
-        constexpr int64_t B = win_bound(Win<NB, 0>::B1);
+        constexpr int64_t B = i32_bound(Win<NB, 0>::B1, L::FIRST);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) load(r, xr[r], xi[r]);
+        for (int r = 0; r < 16; ++r) load(L(), r, xr[r], xi[r]);
         WinTw w, w1;
         bool ok = load_tw32<L, NB, 0>(w, tw, low_bits<L, NB, 0>(t, s, c0), s, logn);
         bool ok1 = true;
@@ -582,23 +427,70 @@ __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_
             int32_t yr[16], yi[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) yr[r] = (int32_t)xr[r], yi[r] = (int32_t)xi[r];
+            if constexpr (L::STAGED) exchange32<L, NB, 0>(yr, yi, t, sm);
             run_win32<L, NB, 0>(yr, yi, w);
             if (narrow_from<L, NB, 1>(yr, yi, tw, t, s, c0, logn, sm, w1, ok1)) {
+                if constexpr (L::STAGED) exchange32<L, NB, (NB + 3) / 4>(yr, yi, t, sm);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) store(r, (int64_t)yr[r], (int64_t)yi[r]);
+                for (int r = 0; r < 16; ++r) store(L(), r, (int64_t)yr[r], (int64_t)yi[r]);
                 return;
             }
+            narrow = true;
         }
     }
     // nothing has been stored: the int64 path starts again from the source
-    // (keeping the loaded or the int32 values for it would hold 64 registers
-    // across the int32 path, one wave per SIMD fewer)
-    asm volatile("" ::: "memory");
+    // (keeping the values for it across the int32 path would hold 64
+    // registers, one wave per SIMD fewer), except that values which failed
+    // window 0's test are still here where the registers allow it (KEEP)
+    if (!L::KEEP || narrow) {
+        asm volatile("" ::: "memory");
 #pragma unroll
-    for (int r = 0; r < 16; ++r) load(r, xr[r], xi[r]);
-    wide_from<L, NB, 0>(xr, xi, tw, t, s, c0, logn, sm);
+        for (int r = 0; r < 16; ++r) load(typename L::Wide(), r, xr[r], xi[r]);
+    }
+    wide_from<typename L::Wide, NB, 0>(xr, xi, tw, t, s, c0, logn, sm);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) store(r, xr[r], xi[r]);
+    for (int r = 0; r < 16; ++r) store(typename L::Wide(), r, xr[r], xi[r]);
+}
+
+// 4096 consecutive points per workgroup: 16 transforms of 256 points and so
+// on.  Points past the batch load as zero and are not stored.  Staging adds
+// two LDS exchanges to save partial-line requests: always at 32 points (8000
+// transforms 7.3 us against 13.4 without), at 64 from 2^18 points (4000: 7.7
+// against 8.6; 2000: 7.6 against 7.4), at 128 from 2^20 (8192: 10.5 against
+// 10.7; 2000: 8.1 against 7.5); a 256-point transform's 16 lanes cover whole
+// lines as they are.
+constexpr int64_t stage_points(int logn) { return logn == 5 ? 0 : logn == 6 ? 1 << 18 : 1 << 20; }
+
+template <int LOGN, bool STAGED>
+__global__ __launch_bounds__(256) void fft_rows_kernel(const int64_t *sre, const int64_t *sim, int64_t *dre,
+                                                       int64_t *dim, const int64_t *__restrict__ tw, int64_t points) {
+    using L = RowsLay<LOGN, STAGED>;
+    constexpr int NP = (LOGN + 3) / 4;
+    __shared__ uint64_t sm[L::ELEMS];
+    const uint32_t t = threadIdx.x;
+    const int64_t off = (int64_t)blockIdx.x << 12;
+    const uint32_t left = (uint32_t)(points - off < 4096 ? points - off : 4096);   // whole transforms
+    const uint32_t tr = L::template col<0>(t) << LOGN, j = t & ((1u << (LOGN - 4)) - 1u);
+    auto load = [&](auto lay, int r, int64_t &re, int64_t &im) {
+        using Y = decltype(lay);
+        const uint32_t i = Y::STAGED ? (uint32_t)r * 256u + t : tr | (bitrev((uint32_t)r, 4) << (LOGN - 4)) | j;
+        if constexpr (L::KEEP) {   // each point is read once
+            re = i < left ? __builtin_nontemporal_load(sre + off + i) : 0;
+            im = i < left ? __builtin_nontemporal_load(sim + off + i) : 0;
+        } else {
+            re = i < left ? sre[off + i] : 0;
+            im = i < left ? sim[off + i] : 0;
+        }
+    };
+    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](auto lay, int r, int64_t re, int64_t im) {
+        using Y = decltype(lay);
+        const uint32_t i = Y::STAGED ? (uint32_t)r * 256u + t
+                                     : tr | win_pos(L::template label<NP - 1>(t), r, Win<LOGN, NP - 1>::S);
+        if (i < left) {
+            __builtin_nontemporal_store(re, dre + off + i);   // streamed: read by no one here
+            __builtin_nontemporal_store(im, dim + off + i);
+        }
+    });
 }
 
 // One workgroup per transform (in place allowed: a workgroup holds its whole
@@ -612,11 +504,11 @@ __global__ __launch_bounds__(1 << (LOGN - 4)) void fft_block_kernel(const int64_
     __shared__ uint64_t sm[L::ELEMS];
     const uint32_t t = threadIdx.x;
     const int64_t off = (int64_t)blockIdx.x << LOGN;
-    auto load = [&](int r, int64_t &re, int64_t &im) {
+    auto load = [&](auto, int r, int64_t &re, int64_t &im) {
         const uint32_t src = (bitrev((uint32_t)r, 4) << (LOGN - 4)) | t;
         re = sre[off + src], im = sim[off + src];
     };
-    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](int r, int64_t re, int64_t im) {
+    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](auto, int r, int64_t re, int64_t im) {
         const uint32_t pos = win_pos(L::template label<NP - 1>(t), r, Win<LOGN, NP - 1>::S);
         dre[off + pos] = re, dim[off + pos] = im;
     });
@@ -639,11 +531,11 @@ __global__ __launch_bounds__(1 << NB) void fft_cols_kernel(const int64_t *sre, c
     const uint32_t high = FIRST ? 0u : (blk >> (s - 4)) << (s + NB);
     const uint32_t j = t >> 4, c = c0 + (t & 15u);
     const uint32_t base = FIRST ? (bitrev(j, NB - 4) << (logn - NB)) | c : high | (j << (s + 4)) | c;
-    auto load = [&](int r, int64_t &re, int64_t &im) {
+    auto load = [&](auto, int r, int64_t &re, int64_t &im) {
         const uint32_t src = base + (FIRST ? bitrev((uint32_t)r, 4) << (logn - 4) : (uint32_t)r << s);
         re = sre[off + src], im = sim[off + src];
     };
-    run_pass<L, NB>(tw, t, s, c0, logn, sm, load, [&](int r, int64_t re, int64_t im) {
+    run_pass<L, NB>(tw, t, s, c0, logn, sm, load, [&](auto, int r, int64_t re, int64_t im) {
         const uint32_t l = win_pos(L::template label<NP - 1>(t), r, Win<NB, NP - 1>::S);
         const uint32_t cc = c0 + L::template col<NP - 1>(t);
         const uint32_t pos = FIRST ? (bitrev(cc, logn - NB) << NB) | l : high | (l << s) | cc;
@@ -756,7 +648,6 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
     if (batch <= 0) return hipSuccess;
     if (logn < 0 || logn > 30) return hipErrorInvalidValue;
     const int64_t n = (int64_t)1 << logn;
-    const unsigned cap = 256 * 16;   // resident-size grid for the grid-stride kernels
     switch (logn) {
 #define SMALL(LG)                                                                                              \
     case LG:                                                                                                   \
@@ -773,9 +664,19 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
                                LG);                                                                            \
             break;                                                                                             \
         }                                                                                                      \
-        const int64_t fpb = 256 / ((1 << LG) / 16), blocks = (batch + fpb - 1) / fpb;                        \
-        const unsigned grid = (unsigned)(blocks < cap ? blocks : cap);                                         \
-        hipLaunchKernelGGL(fft_lds_kernel<LG>, dim3(grid), dim3(256), 0, s, sre, sim, dre, dim, tw, batch);   \
+        if constexpr (LG >= 10) {                                                                              \
+            hipLaunchKernelGGL(fft_block_kernel<LG>, dim3((unsigned)batch), dim3(1u << (LG - 4)), 0, s, sre, sim,  \
+                               dre, dim, tw);                                                                  \
+        } else {                                                                                               \
+            const int64_t points = batch << LG;                                                                \
+            const dim3 grid((unsigned)((points + 4095) / 4096));                                               \
+            if (LG < 8 && points >= stage_points(LG))                                                           \
+                hipLaunchKernelGGL((fft_rows_kernel<LG, (LG < 8)>), grid, dim3(256), 0, s, sre, sim, dre, dim, tw, \
+                                   points);                                                                    \
+            else                                                                                               \
+                hipLaunchKernelGGL((fft_rows_kernel<LG, false>), grid, dim3(256), 0, s, sre, sim, dre, dim, tw, \
+                                   points);                                                                    \
+        }                                                                                                      \
         break;                                                                                                 \
     }
     LDS(5) LDS(6) LDS(7) LDS(8) LDS(9) LDS(10) LDS(11)

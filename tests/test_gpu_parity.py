@@ -529,17 +529,19 @@ def test_fft_out_of_place_and_path_choice():
         b.free()
 
 
-# Transforms of 4096 points and more: whole transforms per workgroup (4096
-# points; 8192 from a batch of 128) or column passes of 6 to 9 stages (every
+# More than 512 transforms of 32 to 2048 points (the batched kernels, each with
+# a partly filled last workgroup; linear staging at 64 points from 2^18 points
+# and at 128 from 2^20), and of 4096 points and more: whole transforms per
+# workgroup (4096 points; 8192 from a batch of 128) or column passes of 6 to 9 stages (every
 # width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
 # scratch) and out of place.  Amplitudes: Q16; around the bound up to which a
 # four-stage window runs in int32 (about 44.7 million: the window after it then fails
 # its test and the block starts again in int64); +-2^40.
-FFT_LONG = [(12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
+FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (8, 513), (9, 515), (10, 513), (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
 
 
-@pytest.mark.parametrize("logn,batch", FFT_LONG, ids=[f"n{1 << l}_b{b}" for l, b in FFT_LONG])
-def test_fft_long_passes(logn, batch):
+@pytest.mark.parametrize("logn,batch", FFT_PASSES, ids=[f"n{1 << l}_b{b}" for l, b in FFT_PASSES])
+def test_fft_batched_and_long(logn, batch):
     n, s = 1 << logn, M.Stream()
     rng = np.random.default_rng(logn * 977 + batch)
     std = O.fft_twiddles(n)
