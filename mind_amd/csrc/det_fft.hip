@@ -23,7 +23,7 @@
 //                      windows separated by an LDS transpose, one HBM read
 //                      and one write per point (fft_rows_kernel up to 512
 //                      points, fft_block_kernel above; fft_few_kernel for a
-//                      few transforms);
+//                      few transforms of up to 1024 points);
 //   * n >= 4096      : the same up to 8192 points, else passes of 6 to 9
 //                      stages over columns of 16 points (fft_cols_kernel).
 // A window runs in int32 when a bound on its inputs proves that every
@@ -554,23 +554,24 @@ static void launch_cols(const int64_t *sre, const int64_t *sim, int64_t *dre, in
         hipLaunchKernelGGL((fft_cols_kernel<NB, false>), grid, block, 0, st, sre, sim, dre, dim, tw, logn, s, lgb);
 }
 
-// A few transforms (batch <= FEW_BATCH, 32 <= n <= 2048): one workgroup per
-// transform, its points and the twiddle table in LDS, and one butterfly per
-// thread and stage, so the latency of a lone call is logn barrier-separated
-// stages instead of a lane walking its 16 points through every stage (the
-// batched kernel gives a single transform only n / 16 lanes).  Same
-// butterflies, same stage order: same bits.  Loads and stores touch each
-// point once (an in-place call reads all of its transform before writing, at
-// the first barrier).  Measured against the batched kernel (device time,
-// same box): 256 points x1 8.1 -> 4.0 us, x512 9.4 -> 5.3; 2048 points x1
-// 17.0 -> 11.3, x64 19.7 -> 11.7; past 512 transforms the batched kernel's
-// throughput wins (256 points x2048: 9.8 against 14.0 us).
-constexpr int FEW_BATCH = 512;
+// A few transforms (batch <= few_batch(logn), 32 <= n <= 1024): one workgroup
+// per transform, its points and the twiddle table in LDS, and one butterfly
+// per thread and stage, so the latency of a lone call is logn
+// barrier-separated stages instead of a lane walking its 16 points through
+// every stage.  Same butterflies, same stage order: same bits.  Loads and
+// stores touch each point once (an in-place call reads all of its transform
+// before writing, at the first barrier).  Per call, this against the window
+// kernels (with about 7 us of host submission in both): 256 points x16 7.2
+// against 7.2 us (inputs up to 2^40: 7.2 against 9.0), 512 points x128 7.2
+// against 8.3, 1024 points x128 7.5 against 7.2 (7.5 against 9.1), but x512
+// 11.4 against 8.1, and 2048 points x1 11.3 against 7.7, x512 21.0 against
+// 14.9.
+constexpr int few_batch(int logn) { return logn <= 9 ? 512 : logn == 10 ? 256 : 0; }
 
-__global__ __launch_bounds__(1024) void fft_few_kernel(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
+__global__ __launch_bounds__(512) void fft_few_kernel(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
                                                        int64_t *dre, int64_t *dim, const int64_t *__restrict__ tw,
                                                        int logn) {
-    __shared__ int64_t lre[2048], lim[2048], ltw[2048];
+    __shared__ int64_t lre[1024], lim[1024], ltw[1024];
     const int n = 1 << logn, half_n = n >> 1, t = threadIdx.x;
     const size_t base = (size_t)blockIdx.x * n;
     for (int i = t; i < n; i += blockDim.x) {   // bit reversal on the way in
@@ -658,10 +659,9 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
 #undef SMALL
 #define LDS(LG)                                                                                                \
     case LG: {                                                                                                 \
-        if (batch <= FEW_BATCH) {                                                                              \
-            const unsigned threads = (1u << LG) / 2 < 1024 ? (1u << LG) / 2 : 1024;                            \
-            hipLaunchKernelGGL(fft_few_kernel, dim3((unsigned)batch), dim3(threads), 0, s, sre, sim, dre, dim, tw, \
-                               LG);                                                                            \
+        if (batch <= few_batch(LG)) {                                                                          \
+            hipLaunchKernelGGL(fft_few_kernel, dim3((unsigned)batch), dim3((1u << LG) / 2), 0, s, sre, sim, dre, dim, \
+                               tw, LG);                                                                        \
             break;                                                                                             \
         }                                                                                                      \
         if constexpr (LG >= 10) {                                                                              \
@@ -670,7 +670,7 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
         } else {                                                                                               \
             const int64_t points = batch << LG;                                                                \
             const dim3 grid((unsigned)((points + 4095) / 4096));                                               \
-            if (LG < 8 && points >= stage_points(LG))                                                           \
+            if (LG < 8 && points >= stage_points(LG))                                                          \
                 hipLaunchKernelGGL((fft_rows_kernel<LG, (LG < 8)>), grid, dim3(256), 0, s, sre, sim, dre, dim, tw, \
                                    points);                                                                    \
             else                                                                                               \

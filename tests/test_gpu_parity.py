@@ -434,9 +434,9 @@ def _fft_oracle_batch(re, im, tw, logn):
     return out_r, out_i
 
 
-# batch <= 512 with 32 <= n <= 2048 takes the few-transform kernel (one
-# workgroup per transform), larger batches the batched one: both sides of
-# that bound are covered (512 / 513, 1000).
+# batch <= 512 (256 at n = 1024) with 32 <= n <= 1024 takes the few-transform
+# kernel, larger batches the batched ones: both sides of that bound are
+# covered (512 / 513, 1000 here, 256 / 257 below).
 FFT_CASES = [(logn, batch) for logn in range(0, 15) for batch in (1, 3, 37)] + [(8, 1000), (5, 513), (5, 512),
                                                                               (10, 512), (11, 9)]
 
@@ -537,7 +537,7 @@ def test_fft_out_of_place_and_path_choice():
 # scratch) and out of place.  Amplitudes: Q16; around the bound up to which a
 # four-stage window runs in int32 (about 44.7 million: the window after it then fails
 # its test and the block starts again in int64); +-2^40.
-FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (8, 513), (9, 515), (10, 513), (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
+FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (8, 513), (9, 515), (10, 256), (10, 257), (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
 
 
 @pytest.mark.parametrize("logn,batch", FFT_PASSES, ids=[f"n{1 << l}_b{b}" for l, b in FFT_PASSES])
