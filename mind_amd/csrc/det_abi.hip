@@ -520,13 +520,22 @@ int64_t gemm_host(Op op, int64_t a, int64_t b, int64_t c, int64_t m, int64_t k, 
     return get_outputs(ds, pinned, out, 1, s, direct);
 }
 
-// Q16 GEMV over nb vectors on device pointers: groups of up to 8 vectors go
-// to the MFMA kernel when the shape allows it (and nb >= 2), the rest to the
-// one-vector VALU kernel.  `ws` must hold gemv8_workspace_bytes(K) when
-// gemv_ws_need() is non-zero.
+// Q16 GEMV over nb vectors on device pointers, in groups of up to 8: a group
+// goes to the MFMA kernel where the shape allows it and it pays, else to the
+// VALU kernel.  gemv_ws_need() is the workspace of a shape that the MFMA
+// kernel may take, gemv_ws_used() what this call uses of it (0 when every
+// group goes to the VALU kernel).
 size_t gemv_ws_need(const int32_t *W, const int32_t *X, int64_t m, int64_t k, int64_t nb) {
     if (nb < 2 || k == 0 || !det::gemv8_eligible(W, X, (int)m, (int)k)) return 0;
     return det::gemv8_workspace_bytes((int)k);
+}
+
+size_t gemv_ws_used(const int32_t *W, const int32_t *X, int64_t m, int64_t k, int64_t nb) {
+    const size_t need = gemv_ws_need(W, X, m, k, nb);
+    if (!need) return 0;
+    const bool pays = (nb >= 8 && det::gemv8_pays((int)m, (int)k, 8)) ||
+                      (nb % 8 && det::gemv8_pays((int)m, (int)k, (int)(nb % 8)));
+    return pays ? need : 0;
 }
 
 hipError_t gemv_q16_any(const int32_t *W, const int32_t *X, int32_t *Y, int64_t m, int64_t k, int64_t nb, void *ws,
@@ -536,8 +545,9 @@ hipError_t gemv_q16_any(const int32_t *W, const int32_t *X, int32_t *Y, int64_t 
     if (!ws || nb < 2) return det::launch_gemv_q16(W, X, Y, M, K, (int)nb, s);
     for (int64_t b = 0; b < nb; b += 8) {
         const int g = (int)(nb - b < 8 ? nb - b : 8);
-        hipError_t e = g >= 2 ? det::launch_gemv_q16_mfma(W, X + b * k, Y + b * m, M, K, g, ws, s)
-                              : det::launch_gemv_q16(W, X + b * k, Y + b * m, M, K, g, s);
+        hipError_t e = det::gemv8_pays(M, K, g)
+                             ? det::launch_gemv_q16_mfma(W, X + b * k, Y + b * m, M, K, g, ws, s)
+                             : det::launch_gemv_q16(W, X + b * k, Y + b * m, M, K, g, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -574,7 +584,7 @@ int64_t gemv_host(bool q16, int64_t w, int64_t x, int64_t y, int64_t m, int64_t 
     if (k == 0) DET_HIP_CHECK(zero_i32(dy, (size_t)nb * m, s));
     else if (q16) {
         const int32_t *dW = (const int32_t *)io, *dX = (const int32_t *)(io + off_x);
-        const size_t need = gemv_ws_need(dW, dX, m, k, nb);
+        const size_t need = gemv_ws_used(dW, dX, m, k, nb);
         if ((rc = ensure(&ds.ws, &ds.ws_bytes, need))) return rc;
         // the workspace arena is shared with the device-pointer entry points
         // (other streams): start after its last user, then mark this stream
@@ -931,7 +941,7 @@ int64_t det_gemv_q16_ws_dev(const int32_t *w, const int32_t *x, int32_t *y, int6
     if (bad_dims(m, k, nb)) return set_err(DET_ERR_ARG, "dimension out of range [0, 2^31)");
     if (m == 0 || nb == 0) return 0;
     if (!y || ((!w || !x) && k > 0)) return set_err(DET_ERR_ARG, "null device pointer");
-    const size_t need = gemv_ws_need(w, x, m, k, nb);
+    const size_t need = gemv_ws_used(w, x, m, k, nb);
     const bool enough = need && ws && ws_bytes >= 0 && (size_t)ws_bytes >= need;
     DET_HIP_CHECK(gemv_q16_any(w, x, y, m, k, nb, enough ? ws : nullptr, (hipStream_t)stream));
     return 0;
@@ -943,7 +953,7 @@ int64_t det_gemv_q16_dev(const int32_t *w, const int32_t *x, int32_t *y, int64_t
     if (m == 0 || nb == 0) return 0;
     if (!y || ((!w || !x) && k > 0)) return set_err(DET_ERR_ARG, "null device pointer");
     hipStream_t s = (hipStream_t)stream;
-    const size_t need = gemv_ws_need(w, x, m, k, nb);
+    const size_t need = gemv_ws_used(w, x, m, k, nb);
     if (need == 0) {
         DET_HIP_CHECK(gemv_q16_any(w, x, y, m, k, nb, nullptr, s));
         return 0;

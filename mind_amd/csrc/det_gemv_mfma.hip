@@ -351,6 +351,21 @@ bool gemv8_eligible(const int32_t *W, const int32_t *X, int M, int K) {
            ((uintptr_t)W & 15) == 0 && ((uintptr_t)X & 3) == 0;
 }
 
+// Whether this kernel beats the VALU one (det_gemv.hip) for a group of nb
+// vectors.  Its blocks of 64 rows run one per compute unit and take the same
+// time for 2 vectors as for 8, so it needs nearly full rounds of them and
+// enough vectors.  Device time, this against the VALU kernel: 8 vectors, K =
+// 8192: 12288 rows (192 blocks on 256 CUs) 100 against 117 us, 16384 143
+// against 146, but 8192 rows 87 against 81 and 20000 (313 blocks) 207 against
+// 176; K = 1024 19.2 against 25, K = 512 14.6 against 13.3.  4 vectors: 16384
+// rows, K = 16384 180 against 203, K = 8192 143 against 117; 2 vectors
+// 180 against 169.
+bool gemv8_pays(int M, int K, int nb) {
+    const long long cus = cu_count(), blocks = (M + 63) / 64, room = (blocks + cus - 1) / cus * cus;
+    if (nb > 4) return K >= 1024 && blocks * 10 >= room * 7;
+    return nb > 2 && K > 8192 && blocks * 10 >= room * 9;
+}
+
 // X: [nb][K] with nb <= 8, Y: [nb][M].  Requires gemv8_eligible.
 hipError_t launch_gemv_q16_mfma(const int32_t *W, const int32_t *X, int32_t *Y, int M, int K, int nb, void *ws,
                                 hipStream_t s) {

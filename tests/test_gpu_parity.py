@@ -1422,6 +1422,65 @@ def test_gemv_q16_ws_dev(m, k, nb):
     s.destroy()
 
 
+# Every split of a row (16 lanes, one, two and four waves) with a K remainder,
+# on and off the 16-byte grid, and every group of vectors; (11530, 1024): the
+# rows fill 181 of 256 compute units, so groups of 5 or more take the MFMA
+# kernel when they get a workspace.
+GEMV_SPLITS = [(1, 5), (37, 4099), (2047, 130), (2051, 1100), (4097, 1027), (8193, 1030), (8195, 1025), (11530, 1024)]
+
+
+@pytest.mark.parametrize("m,k", GEMV_SPLITS, ids=[f"{m}x{k}" for m, k in GEMV_SPLITS])
+@pytest.mark.parametrize("off", [0, 1], ids=["aligned", "one_element_off"])
+def test_gemv_row_splits(m, k, off):
+    L, s = M.lib(), M.Stream()
+    rng = np.random.default_rng(m * 31 + k + off)
+    W = rng.integers(-(1 << 31), 1 << 31, m * k + off).astype(np.int32)
+    W[rng.integers(0, W.size, 64)] = -(1 << 31)
+    Wi = rng.integers(-32768, 32768, m * k + off).astype(np.int16)
+    Wi[rng.integers(0, Wi.size, 64)] = -32768
+    dW, dWi = M.DeviceBuffer.from_array(W), M.DeviceBuffer.from_array(Wi)
+    for nb in (1, 2, 3, 4, 5, 8, 13):
+        X = rng.integers(-(1 << 31), 1 << 31, nb * k + off).astype(np.int32)
+        dX, dY = M.DeviceBuffer.from_array(X), M.DeviceBuffer(nb * m * 4)
+        want = O.gemv_q16_batched(W[off:], X[off:], m, k, nb).reshape(nb, m)
+        need = L.det_gemv_workspace_bytes(m, k, nb)
+        ws = M.DeviceBuffer(max(need, 256))
+        for have in {0, need}:
+            dY.fill(0xA5), ws.fill(0x5B)
+            note(f"gemv q16 {m}x{k} nb={nb} off={off} ws={have}")
+            M.check(L.det_gemv_q16_ws_dev(dW.ptr + 4 * off, dX.ptr + 4 * off, dY.ptr, m, k, nb, ws.ptr, have, s.ptr))
+            s.sync()
+            np.testing.assert_array_equal(dY.to_array(np.int32, (nb, m)), want)
+        for b in (dX, dY, ws):
+            b.free()
+    xi = rng.integers(-32768, 32768, k + off).astype(np.int16)
+    dx, dy = M.DeviceBuffer.from_array(xi), M.DeviceBuffer(m * 4)
+    dy.fill(0xA5)
+    note(f"gemv i16 {m}x{k} off={off}")
+    M.check(L.det_gemv_i16_dev(dWi.ptr + 2 * off, dx.ptr + 2 * off, dy.ptr, m, k, s.ptr))
+    s.sync()
+    np.testing.assert_array_equal(dy.to_array(np.int32, (m,)), O.gemv_i16(Wi[off:], xi[off:], m, k))
+    for b in (dx, dy, dW, dWi):
+        b.free()
+    s.destroy()
+
+
+def test_gemv_q16_residue_fold():
+    """More than 2^16 terms per lane, each with the largest residue (65535):
+    the 32-bit residue sums must be folded in between."""
+    k = 4 * 64 * 4 * ((1 << 14) + 3) + 7
+    W, x = np.full(k, (5 << 16) | 1, np.int32), np.full(k, -1, np.int32)
+    dW, dx, dy, s = M.DeviceBuffer.from_array(W), M.DeviceBuffer.from_array(x), M.DeviceBuffer(4), M.Stream()
+    note(f"gemv q16 1x{k}")
+    M.check(M.lib().det_gemv_q16_dev(dW.ptr, dx.ptr, dy.ptr, 1, k, 1, s.ptr))
+    s.sync()
+    term = (int(W[0]) * -1) >> 16
+    assert int(dy.to_array(np.int32, (1,))[0]) == (k * term + (1 << 31)) % (1 << 32) - (1 << 31)
+    for b in (dW, dx, dy):
+        b.free()
+    s.destroy()
+
+
 @pytest.mark.parametrize("m,k", [(1, 1), (7, 9), (256, 256), (300, 1001), (4096, 4096)])
 def test_gemv_i16_shapes(m, k):
     W, x = O.gen_i16(0xDEADBEEF ^ (m * 3 + k), m * k, k)
