@@ -512,8 +512,10 @@ int64_t gemm_host(Op op, int64_t a, int64_t b, int64_t c, int64_t m, int64_t k, 
     // the workspace arena is shared with the device-pointer entry points:
     // start after its last user, and mark this stream as its next one
     if (need) DET_HIP_CHECK(hipStreamWaitEvent(s, ds.ws_free, 0));
+    // (a few-rows int8 product split in K adds into C with atomics: device memory)
+    const bool adds = op == Op::I8 && det::i8_rows(M, N, K) && det::i8_rows_split(M, N, K) > 1;
     bool direct = false;
-    void *dc = out_ptr(ds, pinned, off_c, bytes_c, &direct);
+    void *dc = out_ptr(ds, pinned && !adds, off_c, bytes_c, &direct);
     if ((rc = gemm_dev(op, io, io + off_b, dc, m, k, n, need ? ds.ws : nullptr, s))) return rc;
     if (need) DET_HIP_CHECK(hipEventRecord(ds.ws_free, s));
     const HostOut out[1] = {{off_c, (void *)c, bytes_c}};

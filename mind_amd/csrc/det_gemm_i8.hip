@@ -1504,6 +1504,7 @@ static void launch_i8_on_grid(const int8_t *A, const int8_t *B, int32_t *C, int 
 hipError_t launch_gemm_i8(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, void *ws,
                           hipStream_t s) {
     using namespace i8g;
+    if (i8_rows(M, N, K)) return launch_gemm_i8_rows(A, B, C, M, N, K, s);
     if (i8_small(M, N, K)) return launch_gemm_i8_small(A, B, C, M, N, K, s);
     const bool aligned = (((uintptr_t)A & 15) == 0) && (((uintptr_t)B & 15) == 0);
     const size_t pad = i8_workspace_bytes(M, N, K, aligned);

@@ -31,7 +31,12 @@ size_t i8_workspace_bytes(int M, int N, int K, bool aligned);
 constexpr long long I8_SMALL_K = 512, I8_SMALL_K_ODD = 4096;
 bool i8_small(int M, int N, int K);
 hipError_t launch_gemm_i8_small(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
-// The same for int16 (v_dot2 kernel), K <= I16_SMALL_K.
+// int8 GEMM with few rows of A (det_gemm_rows.hip): B streamed once, no
+// workspace, any alignment.
+bool i8_rows(int M, int N, int K);
+int i8_rows_split(int M, int N, int K);
+hipError_t launch_gemm_i8_rows(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
+// The direct launch for int16 (v_dot2 kernel), K <= I16_SMALL_K.
 constexpr long long I16_SMALL_K = 4096;
 bool i16_small(int M, int N, int K);
 hipError_t launch_gemm_i16_small(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K,

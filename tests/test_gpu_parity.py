@@ -1100,6 +1100,36 @@ def _offset_buffer(a, off):
     return buf
 
 
+# int8 with up to 64 rows (det_gemm_rows.hip): every group of rows, column tiles
+# that overlap their neighbour, K remainders, K split over workgroups (K >=
+# 3072 and at most 128 units) and not, on and off the 16-byte grid.
+I8_ROWS = [(1, 513, 64), (16, 1000, 65), (17, 3071, 127), (33, 3072, 1030), (49, 4097, 130), (64, 3200, 4100),
+           (2, 8066, 1280), (40, 130, 9000), (64, 96, 8200), (50, 700, 8191), (20, 200, 8300), (3, 5, 20000)]
+
+
+@pytest.mark.parametrize("m,k,n", I8_ROWS, ids=[f"{m}x{k}x{n}" for m, k, n in I8_ROWS])
+def test_gemm_i8_few_rows(m, k, n):
+    L, s = M.lib(), M.Stream()
+    a, b = O.gen_i8(0x2085 ^ (m * 1000003 + k * 1009 + n), m * k, k * n)
+    a[: min(64, a.size)], b[: min(64, b.size)] = -128, -128
+    want = O.gemm_i8(a, b, m, k, n).reshape(m, n)
+    np.testing.assert_array_equal(M.det_matmul_i8(a.reshape(m, k), b.reshape(k, n)), want)
+    for offs in ((0, 0), (1, 3)):
+        da, db = _offset_buffer(a, offs[0]), _offset_buffer(b, offs[1])
+        dc = M.DeviceBuffer(m * n * 4 + 256)
+        for rep in range(2):
+            dc.fill(0xA5)
+            note(f"int8 few rows {m}x{k}x{n} offsets={offs} rep={rep}")
+            M.check(L.det_matmul_i8_dev(da.ptr + offs[0], db.ptr + offs[1], dc.ptr, m, k, n, s.ptr))
+            s.sync()
+            got = dc.to_array(np.int32, (m * n + 64,))
+            np.testing.assert_array_equal(got[:m * n].reshape(m, n), want)
+            assert (got[m * n:] == np.int32(-1515870811)).all()   # nothing written past C
+        for buf in (da, db, dc):
+            buf.free()
+    s.destroy()
+
+
 @pytest.mark.parametrize("m,k,n", RAGGED_I8, ids=[f"{m}x{k}x{n}" for m, k, n in RAGGED_I8])
 @pytest.mark.parametrize("offs", [(0, 0), (1, 3), (8, 4)], ids=["aligned", "off1_3", "off8_4"])
 def test_gemm_i8_ragged_and_misaligned_device_operands(m, k, n, offs):
