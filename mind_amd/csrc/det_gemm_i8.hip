@@ -1433,6 +1433,12 @@ static bool i8_edge_underfills(int M, int N, int K) {
            (long long)(round256(M) / 128) * (long long)(round256(N) / 128) <= cus;
 }
 
+// Shapes on the 16-byte grid that a 128- or 256-row full-tile kernel takes.
+static bool i8_full_tiles(int M, int N, int K) {
+    if (M % 128 || N % 128 || K % 128) return false;
+    return N % 256 == 0 || (long long)(M / 128) * (N / 128) <= cu_count();
+}
+
 size_t i8_workspace_bytes(int M, int N, int K, bool aligned) {
     if (i8_small(M, N, K)) return 0;
     const size_t Mp = round256(M), Kp = round256(K), Np = round256(N);
@@ -1505,10 +1511,14 @@ hipError_t launch_gemm_i8(const int8_t *A, const int8_t *B, int32_t *C, int M, i
                           hipStream_t s) {
     using namespace i8g;
     if (i8_rows(M, N, K)) return launch_gemm_i8_rows(A, B, C, M, N, K, s);
-    if (i8_small(M, N, K)) return launch_gemm_i8_small(A, B, C, M, N, K, s);
     const bool aligned = (((uintptr_t)A & 15) == 0) && (((uintptr_t)B & 15) == 0);
-    const size_t pad = i8_workspace_bytes(M, N, K, aligned);
-    if (i8_fast(A, B, M, N, K) && !(pad && ws)) {
+    const bool small = i8_small(M, N, K);
+    if (small && (K <= I8_SMALL_K || !i8_mid(M, N, K, true))) return launch_gemm_i8_small(A, B, C, M, N, K, s);
+    const size_t pad = small ? 0 : i8_workspace_bytes(M, N, K, aligned);
+    const bool fast = i8_fast(A, B, M, N, K);
+    if (K >= 1 && !(fast && i8_full_tiles(M, N, K)) && i8_mid(M, N, K, fast || (pad && ws)))
+        return launch_gemm_mid(A, B, C, M, N, K, s);
+    if (fast && !(pad && ws)) {
         launch_i8_on_grid(A, B, C, M, N, K, N, M, N, s);
     } else if (pad && ws) {
         const int Mp = (int)round256(M), Kp = (int)round256(K), Np = (int)round256(N);

@@ -374,7 +374,11 @@ size_t i16_workspace_bytes(int M, int N, int K) {
 
 hipError_t launch_gemm_i16(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K, void *ws,
                            hipStream_t s) {
-    if (i16_small(M, N, K)) return launch_gemm_i16_small(A, B, C, M, N, K, s);
+    const bool on_grid = K % 16 == 0 && N % 8 == 0 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+    const bool use_mid = K >= 1 && i16_mid(M, N, K, on_grid), small = i16_small(M, N, K);
+    // (up to K = 512 the tiny-shape kernel is as fast: both at the launch floor)
+    if (use_mid && !(small && K <= 512)) return launch_gemm_mid(A, B, C, M, N, K, s);
+    if (small) return launch_gemm_i16_small(A, B, C, M, N, K, s);
     if (i16x_eligible(M, N, K)) return launch_gemm_i16x(A, B, C, M, N, K, ws, s);
     return launch_limb<int16_t, 2, false>(A, B, C, M, N, K, false, ws, s);
 }

@@ -36,6 +36,15 @@ hipError_t launch_gemm_i8_small(const int8_t *A, const int8_t *B, int32_t *C, in
 bool i8_rows(int M, int N, int K);
 int i8_rows_split(int M, int N, int K);
 hipError_t launch_gemm_i8_rows(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
+// int8 / int16 GEMM in one launch on 64 x 64 tiles (det_gemm_mid.hip): no
+// workspace, any alignment, N >= 64.  i8_mid: for shapes the full-tile kernels
+// do not take as they are, `panels` if the alternative is repacked panels or
+// the edge kernel; i16_mid: `on_grid` if the alternative's prep reads whole
+// 16-byte vectors.
+bool i8_mid(int M, int N, int K, bool panels);
+bool i16_mid(int M, int N, int K, bool on_grid);
+hipError_t launch_gemm_mid(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
+hipError_t launch_gemm_mid(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
 // The direct launch for int16 (v_dot2 kernel), K <= I16_SMALL_K.
 constexpr long long I16_SMALL_K = 4096;
 bool i16_small(int M, int N, int K);

@@ -1100,6 +1100,42 @@ def _offset_buffer(a, off):
     return buf
 
 
+# One-launch 64 x 64 tiles (det_gemm_mid.hip): tiles that overlap their
+# neighbour, row edges, two groups of waves and one (over 256 tiles), K shorter
+# than a step, odd and even step counts, with and without a remainder.
+MID_SHAPES = [(65, 700, 64), (130, 1030, 200), (300, 63, 4000), (200, 2049, 129), (513, 1088, 700), (1100, 130, 1100),
+              (1100, 191, 1090), (70, 1151, 300), (257, 1216, 65), (1000, 33, 1300)]
+
+
+@pytest.mark.parametrize("m,k,n", MID_SHAPES, ids=[f"{m}x{k}x{n}" for m, k, n in MID_SHAPES])
+@pytest.mark.parametrize("op", ["i8", "i16"])
+def test_gemm_mid_tiles(op, m, k, n):
+    L, s = M.lib(), M.Stream()
+    seed = 0x31D ^ (m * 1000003 + k * 1009 + n)
+    a, b = (O.gen_i8 if op == "i8" else O.gen_i16)(seed, m * k, k * n)
+    low = np.iinfo(a.dtype).min
+    a[:: max(1, a.size // 97)], b[:: max(1, b.size // 89)] = low, low
+    want = (O.gemm_i8 if op == "i8" else O.gemm_i16)(a, b, m, k, n).reshape(m, n)
+    code = M.DET_OP_I8 if op == "i8" else M.DET_OP_I16
+    need = L.det_workspace_bytes(code, m, k, n)
+    ws = M.DeviceBuffer(max(need, 256))
+    for off in (0, a.itemsize):
+        da, db = _offset_buffer(a, off), _offset_buffer(b, off)
+        dc = M.DeviceBuffer(m * n * 4 + 256)
+        for have in {need, 0} if op == "i8" else {need}:
+            dc.fill(0xA5), ws.fill(0x5B)
+            note(f"{op} mid tiles {m}x{k}x{n} offset={off} ws={have}")
+            M.check(L.det_matmul_ws_dev(code, da.ptr + off, db.ptr + off, dc.ptr, m, k, n, ws.ptr, have, s.ptr))
+            s.sync()
+            got = dc.to_array(np.int32, (m * n + 64,))
+            np.testing.assert_array_equal(got[:m * n].reshape(m, n), want)
+            assert (got[m * n:] == np.int32(-1515870811)).all()   # nothing written past C
+        for buf in (da, db, dc):
+            buf.free()
+    ws.free()
+    s.destroy()
+
+
 # int8 with up to 64 rows (det_gemm_rows.hip): every group of rows, column tiles
 # that overlap their neighbour, K remainders, K split over workgroups (K >=
 # 3072 and at most 128 units) and not, on and off the 16-byte grid.
