@@ -104,19 +104,34 @@ __global__ __launch_bounds__(THREADS) void small_kernel(const int32_t *__restric
 }  // namespace q16s
 
 // The direct kernel costs K / 4 terms per thread and round of 16x16 tiles
-// over the compute units, plus a fixed cost per workgroup; past
-// Q16_SMALL_ROUNDS rounds or Q16_SMALL_TERMS of K times rounds the limb
-// kernel's prep and extra launches are the cheaper overhead (measured
-// crossovers: 512x1024x512, 4 rounds of K = 1024, still runs faster here;
-// 1024x64x1024, 16 rounds, and 1024x256x1024 do not).  The operand sizes it
-// admits stay far below the 2^31-byte buffer range.
-bool q16_small(int M, int N, int K) {
+// over the compute units, plus a fixed cost per workgroup; past some rounds
+// and terms the limb kernel's prep and extra launches are the cheaper
+// overhead.  The operand sizes admitted stay far below the 2^31-byte buffer
+// range.
+static bool q16_rounds(int M, int N, int K, long long *rounds) {
     if (K < 1) return false;
     const long long tiles = (long long)((M + q16s::TM - 1) / q16s::TM) * ((N + q16s::TN - 1) / q16s::TN);
-    const long long cus = cu_count(), rounds = (tiles + cus - 1) / cus;
-    const long long a_bytes = 4LL * M * K, b_bytes = 4LL * K * N;
-    return rounds <= Q16_SMALL_ROUNDS && rounds * K <= Q16_SMALL_TERMS && a_bytes < (1LL << 31) &&
-           b_bytes < (1LL << 31);
+    const long long cus = cu_count();
+    *rounds = (tiles + cus - 1) / cus;
+    return 4LL * M * K < (1LL << 31) && 4LL * K * N < (1LL << 31);
+}
+
+// Shapes that are far on this side (512x1024x512, 4 rounds of K = 1024, still
+// runs faster here): no workspace is reported for them.
+bool q16_small(int M, int N, int K) {
+    long long rounds = 0;
+    return q16_rounds(M, N, K, &rounds) && rounds <= Q16_SMALL_ROUNDS && rounds * K <= Q16_SMALL_TERMS;
+}
+
+// What the launch goes by: more rounds of a shorter K as well.  Limb path ->
+// here: 448x190x896 (7 rounds) 20.9 -> 13.2 us, 1024x128x512 (8) 17.7 -> 12.7,
+// 700x256x700 (8) 22.1 -> 18.4, 1024x512x300 (5) 26.1 -> 20.7, 512x300x1000 (8)
+// 24.7 -> 23.1, 600x128x1000 (10) 17.3 -> 15.5; but 960x320x640 (10) 25.1 -> 28.4,
+// 640^3 (7) 30.1 -> 33.8, 1000x128x1000 (16) 17.6 -> 24.3.
+bool q16_direct(int M, int N, int K) {
+    long long rounds = 0;
+    if (q16_small(M, N, K)) return true;
+    return q16_rounds(M, N, K, &rounds) && rounds <= 10 && rounds * K <= (rounds <= 8 ? 2600 : 1300);
 }
 
 hipError_t launch_gemm_q16_small(const int32_t *A, const int32_t *B, int32_t *C, int M, int N, int K, bool b_is_t,

@@ -62,6 +62,7 @@ size_t q16x_workspace_bytes(int M, int N, int K);   // the second-generation Q16
 // compute units and rounds times K is at most Q16_SMALL_TERMS.
 constexpr long long Q16_SMALL_ROUNDS = 4, Q16_SMALL_TERMS = 4096;
 bool q16_small(int M, int N, int K);
+bool q16_direct(int M, int N, int K);   // also shapes a workspace is reported for
 hipError_t launch_gemm_q16_small(const int32_t *A, const int32_t *B, int32_t *C, int M, int N, int K, bool b_is_t,
                                  hipStream_t s);
 inline size_t q16_workspace_bytes(int M, int N, int K) {

@@ -1321,6 +1321,20 @@ def test_gemm_q16_multi_tile(gen, shape):
 # 200 x 4160 x 300 (20 tiles), 1000 x 4100 x 33 (16 tiles, one column), 512 x
 # 2048 x 512 (64 tiles, 4 splits of 8 steps); 1000 x 100 x 1000 and 1024 x
 # 128 x 1024 fill the chip (no split; the first ragged in M, N and K).
+# Direct-kernel shapes beyond those that report no workspace (5 to 10 rounds of
+# 16 x 16 tiles), each just inside and just past the rule's limits: the same
+# integers on either route.
+Q_DIRECT_ROUNDS = [(448, 190, 896), (1024, 325, 512), (1024, 326, 512), (600, 130, 1000), (600, 131, 1000),
+                   (1040, 100, 640), (1056, 100, 640)]
+
+
+@pytest.mark.parametrize("m,k,n", Q_DIRECT_ROUNDS, ids=[f"{m}x{k}x{n}" for m, k, n in Q_DIRECT_ROUNDS])
+def test_gemm_q16_direct_rounds(m, k, n):
+    a, b = O.gen_q16_sat(0x9D1 ^ (m * 1000003 + k * 1009 + n), m * k, k * n)
+    note(f"det_matmul_q16 direct rounds {m}x{k}x{n}")
+    np.testing.assert_array_equal(M.det_matmul_q16(a.reshape(m, k), b.reshape(k, n)), O.gemm_q16(a, b, m, k, n))
+
+
 Q_SPLIT = [(7, 5000, 130), (100, 4200, 70), (200, 4160, 300), (1000, 4100, 33), (512, 2048, 512), (1000, 100, 1000),
            (1024, 128, 1024)]
 
