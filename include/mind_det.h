@@ -218,7 +218,7 @@ int64_t det_gemv_q16_dev(const int32_t *w, const int32_t *x, int32_t *y, int64_t
  * the query vectors' MFMA operands, det_gemv_workspace_bytes(m, k, nb) bytes
  * for 16-byte aligned w and 4-byte aligned x (0 when no group of vectors
  * takes the MFMA kernel); it is optional: with less, every vector runs the
- * one-vector kernel.  Its contents need not be initialised. */
+ * kernel that needs none.  Its contents need not be initialised. */
 int64_t det_gemv_workspace_bytes(int64_t m, int64_t k, int64_t nb);
 int64_t det_gemv_q16_ws_dev(const int32_t *w, const int32_t *x, int32_t *y, int64_t m, int64_t k, int64_t nb,
                             void *ws, int64_t ws_bytes, void *stream);
@@ -247,16 +247,18 @@ int64_t det_fft_workspace_bytes(int64_t logn, int64_t batch);
  *    256^3, at any alignment); int16 under the same tile bound with
  *    K <= 4096; Q16 when those tiles fill at most 4 rounds and rounds times
  *    K is at most 4096 (every cube up to 512^3).
- *  - Otherwise int8 needs one only when K or N is not a multiple of 16: its
+ *  - Otherwise int8 may use one only when K or N is not a multiple of 16: its
  *    operands are then repacked into aligned zero-padded panels of
  *    Mp*Kp + Kp*Np bytes (M, K, N rounded up to 256).  int8 operands that
  *    are not 16-byte aligned are repacked the same way when the workspace
  *    given holds that size, and so are aligned shapes of at least 256 rows
  *    and columns that no 128-row kernel takes, whose 256 x 256 tiles would
  *    not fill one round of the GPU and whose padding to multiples of 256 adds
- *    at most 1/8 per dimension (e.g. 1008^3), where the padded panels run
- *    faster.  For int8 the workspace is optional: without it such operands
- *    run a slower byte-load kernel; det_matmul_ws_dev rejects a short
+ *    at most 1/8 per dimension (e.g. 2000^3), where the padded panels run
+ *    faster.  Few rows and mid sizes (M <= 64, 1008^3) are read in place
+ *    whatever the workspace, and so are some int16 and Q16 shapes that a
+ *    workspace is reported for.  For int8 the workspace is optional: without
+ *    it such operands run a slower kernel; det_matmul_ws_dev rejects a short
  *    workspace only for int16 / Q16.
  *  - The figure holds for the current device: the rules above and the K
  *    split of mid-size Q16 grids (which keeps its partial sums in the
