@@ -49,7 +49,7 @@ struct Q16 {
     typedef int32_t T;
     static constexpr int PER = 4;   // elements per vector
     struct Op { v4i32 v; v2u16 lo[2]; };
-    struct Acc { long long s; uint32_t r; };
+    struct Acc { unsigned long long s; uint32_t r; };   // s mod 2^64
     static __device__ __forceinline__ Acc zero() { return {0, 0}; }
     static __device__ __forceinline__ Op op(v4i32 v) {
         Op o;
@@ -58,24 +58,28 @@ struct Q16 {
         o.lo[1] = __builtin_bit_cast(v2u16, __builtin_amdgcn_perm((uint32_t)v.w, (uint32_t)v.z, 0x05040100u));
         return o;
     }
+    // two products of the type's lowest value already reach 2^63: unsigned sums
+    static __device__ __forceinline__ unsigned long long prod(T w, T x) {
+        return (unsigned long long)((long long)w * x);
+    }
     static __device__ __forceinline__ void add(Acc &a, const Op &w, const Op &x) {
         const v2u16 one = {1, 1};
-        a.s += (long long)w.v.x * x.v.x;
-        a.s += (long long)w.v.y * x.v.y;
-        a.s += (long long)w.v.z * x.v.z;
-        a.s += (long long)w.v.w * x.v.w;
+        a.s += prod(w.v.x, x.v.x);
+        a.s += prod(w.v.y, x.v.y);
+        a.s += prod(w.v.z, x.v.z);
+        a.s += prod(w.v.w, x.v.w);
         a.r = __builtin_amdgcn_udot2(w.lo[0] * x.lo[0], one, a.r, false);
         a.r = __builtin_amdgcn_udot2(w.lo[1] * x.lo[1], one, a.r, false);
     }
     static __device__ __forceinline__ void add1(Acc &a, T w, T x) {
-        a.s += (long long)w * x;
+        a.s += prod(w, x);
         a.r += ((uint32_t)w * (uint32_t)x) & 0xffffu;
     }
     // residue sums stay below 2^32 for 2^14 vectors (2^16 terms below 2^16)
     static constexpr int FOLD = 1 << 14;
-    static __device__ __forceinline__ void fold(Acc &a) { a.s -= (long long)a.r, a.r = 0; }
+    static __device__ __forceinline__ void fold(Acc &a) { a.s -= a.r, a.r = 0; }
     typedef unsigned long long Sum;
-    static __device__ __forceinline__ Sum sum(const Acc &a) { return (Sum)a.s - a.r; }
+    static __device__ __forceinline__ Sum sum(const Acc &a) { return a.s - a.r; }
     static __device__ __forceinline__ int32_t out(Sum v) { return (int32_t)(uint32_t)(v >> 16); }
 };
 

@@ -10,6 +10,8 @@ the library's own device flags (hipcc cross-compiles; no GPU needed).
 2. Scalar memory is only read: every scalar instruction is an arithmetic or
    control one, or a scalar load.  Stores go through the vector memory path
    only.
+3. Sums that have to wrap are unsigned in the source: signed overflow is
+   undefined and the build has no -fwrapv.
 
 It is a CPU test: it never needs a GPU."""
 import concurrent.futures as cf
@@ -79,3 +81,26 @@ def test_no_scalar_cache_writes(instructions):
              if t.startswith("s_") and not SCALAR.fullmatch(t.split()[0])}
     assert not found, found
     assert sum(len(v) for v in instructions.values()) > 10000   # the kernels were really compiled
+
+
+# file: (mangled) functions with 64-bit sums that may leave int64's range
+WRAPPING = {"det_gemv.hip": "_ZN3det4gemv3Q16"}
+
+
+@pytest.mark.parametrize("src", sorted(WRAPPING))
+def test_wrapping_sums_are_unsigned(src, tmp_path):
+    """In the unoptimised IR, where clang marks signed sums `nsw`."""
+    out = str(tmp_path / "x.ll")
+    r = subprocess.run([B.HIPCC, *B.DEVICE_FLAGS, "--cuda-device-only", "-S", "-emit-llvm", "-Xclang",
+                        "-disable-llvm-passes", os.path.join(B.CSRC, src), "-o", out],
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    seen, inside = set(), None
+    for line in open(out):
+        if line.startswith("define "):
+            m = re.search(r"@(" + WRAPPING[src] + r"\w*)\(", line)
+            inside = m and m.group(1)
+            seen |= {inside} - {None}
+        elif inside:
+            assert not re.search(r"= (add|sub) nsw i64", line), (inside, line)
+    assert seen
