@@ -150,23 +150,31 @@ __global__ __launch_bounds__(256) void fft_small_kernel(const int64_t *__restric
 // 104 in int32, so the arithmetic matters as much as the stream.  A window
 // therefore runs in int32 whenever its inputs and twiddles allow it
 // (i32_bound).  The test is repeated at each window, so only the window's own
-// growth has to be allowed for; when a test fails the block starts again in
-// int64 (nothing is stored before the last window).  Same butterflies, same
-// stage order, same integers on either path.
+// growth has to be allowed for; when a test fails the block goes on in int64
+// from that window (RESUME: the kernels that hold whole transforms), or starts
+// again from the source (column passes, where going on costs 5% of the int32
+// path: 16 x 2^16 points 27.8 -> 29.2 us; nothing is stored before the last
+// window).  Same butterflies, same stage order, same integers on either path.
 // Device time per call, out of place, inputs within 2^16 (before: windows of
 // the short transforms in one kernel with an all-or-nothing int32 test that
 // left n >= 1024 in int64; one global-memory pass per 4 stages beyond, whose
 // first pass gathered single 8-byte points):
-//   65536 x 256 points 102.7 -> 95 us (5.6 TB/s; a large copy reaches 5.2),
-//   32768 x 512 150 -> 97, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 116,
-//   100000 x 64 88 -> 41-45, 100000 x 128 104 -> 76, 300000 x 32 355 -> 58-61;
+//   65536 x 256 points 102.7 -> 94 us (5.7 TB/s; a large copy reaches 5.2),
+//   32768 x 512 150 -> 100, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 116,
+//   100000 x 64 80 -> 38, 100000 x 128 102 -> 68, 300000 x 32 335 -> 55;
+//   up to 4% slower where the launch is most of the time (513 x 64 6.1 -> 6.3),
+//   and 9000 - 12000 x 128 9.5 - 11.0 -> 10.3 - 11.3;
 //   16 x 2^16 points 86.1 -> 25.5 (34 MB read and written once: 6.6 us at the
 //   copy rate; the two passes wait for memory, then compute, with one workgroup
 //   per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
 //   61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7.
-// Inputs within 2^40 (int64): 65536 x 256 114 -> 115, 32768 x 512 192 -> 133,
-//   13594 x 1024 231 -> 136, 8192 x 2048 302 -> 174, 100000 x 64 83 -> 58,
-//   16 x 2^16 86 -> 33.7.
+// Inputs within 2^40 (int64): 65536 x 256 114 -> 117, 32768 x 512 190 -> 134,
+//   13594 x 1024 231 -> 136, 8192 x 2048 302 -> 173, 100000 x 64 73 -> 50,
+//   100000 x 128 104 -> 96, 12000 x 128 13.8 -> 14.5, 16 x 2^16 86 -> 36.
+// Inputs up to 2^25, where a later window's test fails (before: int64
+// throughout; restarting; going on): 65536 x 256 114, 162, 109 us, 8192 x 256
+// 16.3, 20.0, 14.5, 600 x 512 12.5, 14.8, 10.9, 300 x 1024 10.8, 12.2, 9.5,
+// 16 x 2048 11.6, 13.2, 10.2 (2^22: 11.6, 15.0, 9.0).
 // Window P of NB bits: first bit of its 4 registers, and the stages it runs.
 template <int NB, int P>
 struct Win {
@@ -179,7 +187,7 @@ struct Win {
 template <int NB>
 struct BlockLay {   // a whole transform, one column
     static constexpr int THREADS = 1 << (NB - 4), ELEMS = 1 << NB;
-    static constexpr bool FIRST = true, STAGED = false, KEEP = false;
+    static constexpr bool FIRST = true, STAGED = false, KEEP = false, RESUME = true;
     using Wide = BlockLay;
     // window 0 takes its labels bit-reversed: neighbouring threads then load
     // neighbouring source points
@@ -204,7 +212,9 @@ struct RowsLay {   // 4096 consecutive points: 2^(12 - NB) whole short transform
     // STAGED: loads and stores are linear and go through LDS (below 256 points
     // a window's lanes cover less than a 128-byte line of each transform).
     // The int64 path, 16 bytes a point, is staged below 128 points only.
-    static constexpr bool STAGED = STAGED_, KEEP = !STAGED;
+    // KEEP: inputs that fail window 0's test stay in registers (same layout;
+    // 600 x 32 points in +-2^40 9.9 us read again, 8.7 kept).
+    static constexpr bool STAGED = STAGED_, KEEP = !STAGED || NB < 7, RESUME = true;
     using Wide = RowsLay<NB, STAGED_ && (NB < 7)>;
     template <int P>
     static __device__ __forceinline__ uint32_t label(uint32_t t) {
@@ -229,7 +239,7 @@ struct RowsLay {   // 4096 consecutive points: 2^(12 - NB) whole short transform
 template <int NB, bool FIRST_>
 struct ColsLay {   // 2^NB positions of 16 columns
     static constexpr int THREADS = 1 << NB, ELEMS = 16 << NB, NP = (NB + 3) / 4;
-    static constexpr bool FIRST = FIRST_, STAGED = false, KEEP = false;
+    static constexpr bool FIRST = FIRST_, STAGED = false, KEEP = false, RESUME = false;
     using Wide = ColsLay;
     // the first pass stores runs of consecutive positions of one column, so
     // its last window has lanes along the positions; else lanes run along
@@ -363,10 +373,11 @@ __device__ __forceinline__ uint32_t low_bits(uint32_t t, int s, uint32_t c0) {
 // (L::FIRST) w holds window P's (w_ok: all small), loaded one window ahead;
 // in later passes that would cost the second wave per SIMD (16 transforms of
 // 2^16 25.8 us instead of 27, 32 of them 41.9 instead of 38.6), so they are
-// loaded here.  Returns false when a window's test fails.
+// loaded here.  Returns the window whose test failed (the values are then its
+// inputs), or NP when all have run.
 template <class L, int NB, int P>
-__device__ __forceinline__ bool narrow_from(int32_t (&yr)[16], int32_t (&yi)[16], const int64_t *__restrict__ tw,
-                                            uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, WinTw &w, bool w_ok) {
+__device__ __forceinline__ int narrow_from(int32_t (&yr)[16], int32_t (&yi)[16], const int64_t *__restrict__ tw,
+                                           uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, WinTw &w, bool w_ok) {
     if constexpr (P < (NB + 3) / 4) {
         constexpr int32_t B = i32_bound(Win<NB, P>::B1 - Win<NB, P>::B0, false);
         WinTw wn;
@@ -380,42 +391,50 @@ __device__ __forceinline__ bool narrow_from(int32_t (&yr)[16], int32_t (&yi)[16]
             hi = max(max(hi, yr[r]), yi[r]);
             lo = min(min(lo, yr[r]), yi[r]);
         }
-        if (!block_all(w_ok && hi <= B && lo >= -B)) return false;
+        const bool fits = block_all(w_ok && hi <= B && lo >= -B);
+        if (!L::RESUME && !fits) return P;
         exchange32<L, NB, P>(yr, yi, t, sm);
+        if (!fits) return P;
         run_win32<L, NB, P>(yr, yi, w);
         return narrow_from<L, NB, P + 1>(yr, yi, tw, t, s, c0, logn, sm, wn, wn_ok);
     }
-    return true;
+    return P;
 }
 
+// Windows P.. of the int64 path, or those from `from` on (uniform, at least P),
+// whose inputs x then holds.
 template <class L, int NB, int P>
 __device__ __forceinline__ void wide_from(int64_t (&xr)[16], int64_t (&xi)[16], const int64_t *__restrict__ tw,
-                                          uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm) {
-    if constexpr (P < (NB + 3) / 4) {
-        if constexpr (P > 0 || L::STAGED) {
-            exchange<L, NB, P>(xr, t, (int64_t *)sm);
-            exchange<L, NB, P>(xi, t, (int64_t *)sm);
+                                          uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, int from) {
+    constexpr int NP = (NB + 3) / 4;
+    if constexpr (P < NP) {
+        if (NP == 2 || from <= P) {
+            if ((P > 0 || L::STAGED) && from < P) {
+                exchange<L, NB, P>(xr, t, (int64_t *)sm);
+                exchange<L, NB, P>(xi, t, (int64_t *)sm);
+            }
+            run_win64<L, NB, P>(xr, xi, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
         }
-        run_win64<L, NB, P>(xr, xi, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
-        wide_from<L, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm);
+        wide_from<L, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm, from);
     } else if constexpr (L::STAGED) {
         exchange<L, NB, P>(xr, t, (int64_t *)sm);
         exchange<L, NB, P>(xi, t, (int64_t *)sm);
     }
 }
 
-// All NB stages [s, s + NB): load(layout, r, re, im) gives window 0's points
-// (twice if need be), store(layout, r, re, im) takes the last window's (linear
-// order on both sides where staged).
+// All NB stages [s, s + NB): load(layout, t, r, re, im) gives window 0's
+// points (twice if need be), store(layout, t, r, re, im) takes the last
+// window's (linear order on both sides where staged).
 template <class L, int NB, typename LD, typename ST>
 __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_t t, int s, uint32_t c0, int logn,
                                          uint64_t *sm, LD &&load, ST &&store) {
+    constexpr int NP = (NB + 3) / 4;
     int64_t xr[16], xi[16];
-    bool narrow = false;
+    int from = 0;   // the window at which the int64 path takes over
     {
         constexpr int64_t B = i32_bound(Win<NB, 0>::B1, L::FIRST);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) load(L(), r, xr[r], xi[r]);
+        for (int r = 0; r < 16; ++r) load(L(), t, r, xr[r], xi[r]);
         WinTw w, w1;
         bool ok = load_tw32<L, NB, 0>(w, tw, low_bits<L, NB, 0>(t, s, c0), s, logn);
         bool ok1 = true;
@@ -429,37 +448,49 @@ __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_
             for (int r = 0; r < 16; ++r) yr[r] = (int32_t)xr[r], yi[r] = (int32_t)xi[r];
             if constexpr (L::STAGED) exchange32<L, NB, 0>(yr, yi, t, sm);
             run_win32<L, NB, 0>(yr, yi, w);
-            if (narrow_from<L, NB, 1>(yr, yi, tw, t, s, c0, logn, sm, w1, ok1)) {
-                if constexpr (L::STAGED) exchange32<L, NB, (NB + 3) / 4>(yr, yi, t, sm);
+            from = narrow_from<L, NB, 1>(yr, yi, tw, t, s, c0, logn, sm, w1, ok1);
+            if (from == NP) {
+                if constexpr (L::STAGED) exchange32<L, NB, NP>(yr, yi, t, sm);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) store(L(), r, (int64_t)yr[r], (int64_t)yi[r]);
+                for (int r = 0; r < 16; ++r) store(L(), t, r, (int64_t)yr[r], (int64_t)yi[r]);
                 return;
             }
-            narrow = true;
+            if constexpr (L::RESUME)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) xr[r] = yr[r], xi[r] = yi[r];
         }
     }
-    // nothing has been stored: the int64 path starts again from the source
-    // (keeping the values for it across the int32 path would hold 64
-    // registers, one wave per SIMD fewer), except that values which failed
-    // window 0's test are still here where the registers allow it (KEEP)
-    if (!L::KEEP || narrow) {
+    using W = typename L::Wide;
+    if constexpr (L::RESUME) {
+        // LDS positions and addresses of its own: sharing the int32 path's
+        // would hold them in registers across it
+        asm volatile("" : "+v"(t));
+        if (from) {   // W's labels are L's from window 1 on
+            wide_from<W, NB, 1>(xr, xi, tw, t, s, c0, logn, sm, from);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) store(W(), t, r, xr[r], xi[r]);
+            return;
+        }
+    }
+    if (!L::KEEP) {
         asm volatile("" ::: "memory");
 #pragma unroll
-        for (int r = 0; r < 16; ++r) load(typename L::Wide(), r, xr[r], xi[r]);
+        for (int r = 0; r < 16; ++r) load(W(), t, r, xr[r], xi[r]);
     }
-    wide_from<typename L::Wide, NB, 0>(xr, xi, tw, t, s, c0, logn, sm);
+    wide_from<W, NB, 0>(xr, xi, tw, t, s, c0, logn, sm, -1);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) store(typename L::Wide(), r, xr[r], xi[r]);
+    for (int r = 0; r < 16; ++r) store(W(), t, r, xr[r], xi[r]);
 }
 
 // 4096 consecutive points per workgroup: 16 transforms of 256 points and so
 // on.  Points past the batch load as zero and are not stored.  Staging adds
 // two LDS exchanges to save partial-line requests: always at 32 points (8000
-// transforms 7.3 us against 13.4 without), at 64 from 2^18 points (4000: 7.7
-// against 8.6; 2000: 7.6 against 7.4), at 128 from 2^20 (8192: 10.5 against
-// 10.7; 2000: 8.1 against 7.5); a 256-point transform's 16 lanes cover whole
+// transforms 7.0 us against 10.5 without; 2000 6.8 against 8.1), at 64 from
+// 2^18 points (8000: 7.4 against 9.7), at 128 from 5 x 2^18 (16000: 12.4
+// against 14.8; 8192: 9.0 against 9.1, but inputs past 2^26, read again in the
+// other order, 12.1 against 10.7); a 256-point transform's 16 lanes cover whole
 // lines as they are.
-constexpr int64_t stage_points(int logn) { return logn == 5 ? 0 : logn == 6 ? 1 << 18 : 1 << 20; }
+constexpr int64_t stage_points(int logn) { return logn == 5 ? 0 : logn == 6 ? 1 << 18 : 5 << 18; }
 
 template <int LOGN, bool STAGED>
 __global__ __launch_bounds__(256) void fft_rows_kernel(const int64_t *sre, const int64_t *sim, int64_t *dre,
@@ -467,14 +498,13 @@ __global__ __launch_bounds__(256) void fft_rows_kernel(const int64_t *sre, const
     using L = RowsLay<LOGN, STAGED>;
     constexpr int NP = (LOGN + 3) / 4;
     __shared__ uint64_t sm[L::ELEMS];
-    const uint32_t t = threadIdx.x;
     const int64_t off = (int64_t)blockIdx.x << 12;
     const uint32_t left = (uint32_t)(points - off < 4096 ? points - off : 4096);   // whole transforms
-    const uint32_t tr = L::template col<0>(t) << LOGN, j = t & ((1u << (LOGN - 4)) - 1u);
-    auto load = [&](auto lay, int r, int64_t &re, int64_t &im) {
+    auto load = [&](auto lay, uint32_t t, int r, int64_t &re, int64_t &im) {
         using Y = decltype(lay);
+        const uint32_t tr = L::template col<0>(t) << LOGN, j = t & ((1u << (LOGN - 4)) - 1u);
         const uint32_t i = Y::STAGED ? (uint32_t)r * 256u + t : tr | (bitrev((uint32_t)r, 4) << (LOGN - 4)) | j;
-        if constexpr (L::KEEP) {   // each point is read once
+        if constexpr (L::KEEP && !L::STAGED) {   // each point is read once
             re = i < left ? __builtin_nontemporal_load(sre + off + i) : 0;
             im = i < left ? __builtin_nontemporal_load(sim + off + i) : 0;
         } else {
@@ -482,8 +512,9 @@ __global__ __launch_bounds__(256) void fft_rows_kernel(const int64_t *sre, const
             im = i < left ? sim[off + i] : 0;
         }
     };
-    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](auto lay, int r, int64_t re, int64_t im) {
+    run_pass<L, LOGN>(tw, threadIdx.x, 0, 0, LOGN, sm, load, [&](auto lay, uint32_t t, int r, int64_t re, int64_t im) {
         using Y = decltype(lay);
+        const uint32_t tr = L::template col<0>(t) << LOGN;
         const uint32_t i = Y::STAGED ? (uint32_t)r * 256u + t
                                      : tr | win_pos(L::template label<NP - 1>(t), r, Win<LOGN, NP - 1>::S);
         if (i < left) {
@@ -502,13 +533,12 @@ __global__ __launch_bounds__(1 << (LOGN - 4)) void fft_block_kernel(const int64_
     using L = BlockLay<LOGN>;
     constexpr int NP = (LOGN + 3) / 4;
     __shared__ uint64_t sm[L::ELEMS];
-    const uint32_t t = threadIdx.x;
     const int64_t off = (int64_t)blockIdx.x << LOGN;
-    auto load = [&](auto, int r, int64_t &re, int64_t &im) {
+    auto load = [&](auto, uint32_t t, int r, int64_t &re, int64_t &im) {
         const uint32_t src = (bitrev((uint32_t)r, 4) << (LOGN - 4)) | t;
         re = sre[off + src], im = sim[off + src];
     };
-    run_pass<L, LOGN>(tw, t, 0, 0, LOGN, sm, load, [&](auto, int r, int64_t re, int64_t im) {
+    run_pass<L, LOGN>(tw, threadIdx.x, 0, 0, LOGN, sm, load, [&](auto, uint32_t t, int r, int64_t re, int64_t im) {
         const uint32_t pos = win_pos(L::template label<NP - 1>(t), r, Win<LOGN, NP - 1>::S);
         dre[off + pos] = re, dim[off + pos] = im;
     });
@@ -525,17 +555,17 @@ __global__ __launch_bounds__(1 << NB) void fft_cols_kernel(const int64_t *sre, c
     using L = ColsLay<NB, FIRST>;
     constexpr int NP = (NB + 3) / 4;
     __shared__ uint64_t sm[L::ELEMS];
-    const uint32_t t = threadIdx.x, blk = blockIdx.x & ((1u << lgb) - 1u);
+    const uint32_t blk = blockIdx.x & ((1u << lgb) - 1u);
     const int64_t off = (int64_t)(blockIdx.x >> lgb) << logn;
     const uint32_t c0 = (FIRST ? blk : blk & ((1u << (s - 4)) - 1u)) << 4;
     const uint32_t high = FIRST ? 0u : (blk >> (s - 4)) << (s + NB);
-    const uint32_t j = t >> 4, c = c0 + (t & 15u);
-    const uint32_t base = FIRST ? (bitrev(j, NB - 4) << (logn - NB)) | c : high | (j << (s + 4)) | c;
-    auto load = [&](auto, int r, int64_t &re, int64_t &im) {
+    auto load = [&](auto, uint32_t t, int r, int64_t &re, int64_t &im) {
+        const uint32_t j = t >> 4, c = c0 + (t & 15u);
+        const uint32_t base = FIRST ? (bitrev(j, NB - 4) << (logn - NB)) | c : high | (j << (s + 4)) | c;
         const uint32_t src = base + (FIRST ? bitrev((uint32_t)r, 4) << (logn - 4) : (uint32_t)r << s);
         re = sre[off + src], im = sim[off + src];
     };
-    run_pass<L, NB>(tw, t, s, c0, logn, sm, load, [&](auto, int r, int64_t re, int64_t im) {
+    run_pass<L, NB>(tw, threadIdx.x, s, c0, logn, sm, load, [&](auto, uint32_t t, int r, int64_t re, int64_t im) {
         const uint32_t l = win_pos(L::template label<NP - 1>(t), r, Win<NB, NP - 1>::S);
         const uint32_t cc = c0 + L::template col<NP - 1>(t);
         const uint32_t pos = FIRST ? (bitrev(cc, logn - NB) << NB) | l : high | (l << s) | cc;

@@ -531,13 +531,14 @@ def test_fft_out_of_place_and_path_choice():
 
 # More than 512 transforms of 32 to 2048 points (the batched kernels, each with
 # a partly filled last workgroup; linear staging at 64 points from 2^18 points
-# and at 128 from 2^20), and of 4096 points and more: whole transforms per
+# and at 128 from 5 x 2^18), and of 4096 points and more: whole transforms per
 # workgroup (4096 points; 8192 from a batch of 128) or column passes of 6 to 9 stages (every
 # width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
-# scratch) and out of place.  Amplitudes: Q16; around the bound up to which a
-# four-stage window runs in int32 (about 44.7 million: the window after it then fails
-# its test and the block starts again in int64); +-2^40.
-FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (8, 513), (9, 515), (10, 256), (10, 257), (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
+# scratch) and out of place.  Amplitudes: Q16; about 44.7 million, which passes
+# the first window's test and fails a later one's (the block then goes on in
+# int64, or starts again); +-2^40.
+FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (7, 10243), (8, 513), (9, 515), (10, 256), (10, 257),
+              (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
 
 
 @pytest.mark.parametrize("logn,batch", FFT_PASSES, ids=[f"n{1 << l}_b{b}" for l, b in FFT_PASSES])
@@ -571,6 +572,112 @@ def test_fft_batched_and_long(logn, batch):
         assert np.array_equal(sim.to_array(np.int64, re.shape)[sel], want[1])
         for b in (sre, sim, dre, dim_, dtw):
             b.free()
+    s.destroy()
+
+
+# ------------------------------------------------ FFT: the int32 windows' bounds
+# A window of four stages runs in int32 when its inputs are within
+# bound(stages) (det_fft.hip); inputs at the bound and one past it, on either
+# side, at every window of every kernel, with signs that make a result as large
+# as such inputs allow; and the smallest such inputs that overflow int32.
+
+def _i32_bound(stages, peeled):
+    g = 1.0
+    for i in range(stages):
+        g *= 2.0 if peeled and i == 0 else 2.4143
+    return int((2147483647.0 / g - 4.0) / 1.41422)
+
+
+def _window_gains(tw, logn, first, stages):
+    """Result r of stages [first, first + stages) on 2^stages points p << first:
+    sum of gains[r, p] x[p] (without the floors)."""
+    g = np.eye(1 << stages, dtype=complex)
+    for b in range(stages):
+        for p in range(1 << stages):
+            if p & (1 << b):
+                continue
+            k = ((p & ((1 << b) - 1)) << first) << (logn - 1 - b - first)
+            w = complex(tw[2 * k], tw[2 * k + 1]) / 65536 if first + b else 1.0
+            q = p | (1 << b)
+            g[p], g[q] = g[p] + w * g[q], g[p] - w * g[q]
+    return g
+
+
+def _largest(gains):
+    """Signs (real, imaginary) of the inputs for the largest component."""
+    size = np.abs(gains.real).sum(1) + np.abs(gains.imag).sum(1)
+    c = gains[int(np.argmax(size))]
+    return np.where(c.real < 0, -1, 1), np.where(c.imag < 0, 1, -1), float(size.max())
+
+
+def _at_level(logn, level, stages, signs, lo, hi):
+    """Inputs whose values, once the stages below `level` have run, are lo or hi
+    by `signs` at the positions that are multiples of 2^level (a group's sum),
+    and small elsewhere (its first input's rest, spread)."""
+    n, out = 1 << logn, []
+    rev = np.array([int(format(p, f"0{logn}b")[::-1], 2) for p in range(n)])
+    for s in signs:
+        v = np.where(np.tile(s, n >> (level + stages)) > 0, hi, lo).astype(np.int64)
+        u = v >> level
+        x = np.repeat(u, 1 << level)
+        x[:: 1 << level] += v - (u << level)
+        y = np.empty(n, np.int64)
+        y[rev] = x
+        out.append(y)
+    return out
+
+
+def _check_fft(re, im, tw, logn, batch, s, what):
+    n = 1 << logn
+    want = _fft_oracle_batch(re[None], im[None], tw, logn)
+    bufs = [M.DeviceBuffer.from_array(np.tile(x, batch)) for x in (re, im)]
+    bufs += [M.DeviceBuffer.from_array(tw), M.DeviceBuffer(batch * n * 8), M.DeviceBuffer(batch * n * 8)]
+    note(f"fft bounds n={n} batch={batch} {what}")
+    M.check(M.lib().det_fft_q16_oop_dev(bufs[0].ptr, bufs[1].ptr, bufs[3].ptr, bufs[4].ptr, bufs[2].ptr, logn, n,
+                                        batch, s.ptr))
+    s.sync()
+    for b, w in zip(bufs[3:], want):
+        assert (b.to_array(np.int64, (batch, n)) == w).all(), what
+    for b in bufs:
+        b.free()
+
+
+# (logn, batch, stages of each pass): short transforms, staged and not; a
+# transform per workgroup; column passes
+FFT_BOUNDS = [(5, 600, [5]), (6, 600, [6]), (6, 4100, [6]), (7, 600, [7]), (7, 10300, [7]), (8, 600, [8]),
+              (9, 600, [9]), (10, 300, [10]), (11, 3, [11]), (12, 2, [12]), (13, 128, [13]), (13, 2, [7, 6]),
+              (15, 1, [8, 7]), (17, 1, [9, 8])]
+
+
+@pytest.mark.parametrize("logn,batch,passes", FFT_BOUNDS, ids=[f"n{1 << l}_b{b}" for l, b, _ in FFT_BOUNDS])
+def test_fft_int32_window_bounds(logn, batch, passes):
+    n, s, tw = 1 << logn, M.Stream(), O.fft_twiddles(1 << logn)
+    level = 0
+    for nb in passes:
+        for first in range(0, nb, 4):
+            stages = min(4, nb - first)
+            bound = _i32_bound(stages, level + first == 0)
+            re, im, gain = _largest(_window_gains(tw, logn, level + first, stages))
+            past = int(2**31 * 1.01 / gain)
+            for lo, hi in ((-bound, bound), (-bound - 1, bound), (-bound, bound + 1), (-past, past)):
+                x = _at_level(logn, level + first, stages, (re, im), lo, hi)
+                _check_fft(*x, tw, logn, batch, s, f"window at {level + first}, {lo}..{hi}")
+        level += nb
+    # the largest twiddles that a window takes, sqrt 2 in magnitude: results
+    # of the first window come close to 2^31
+    rng = np.random.default_rng(logn)
+    bound = _i32_bound(4, True)
+    tables = [np.where(rng.integers(0, 2, n), 65536, -65536).astype(np.int64) for _ in range(64)]
+    best = max((_largest(_window_gains(t, logn, 0, 4)) + (t,) for t in tables), key=lambda v: v[2])
+    assert best[2] * bound > 0.7 * 2**31
+    past = int(2**31 * 1.01 / best[2])
+    for lo, hi in ((-bound, bound), (-bound - 1, bound), (-bound, bound + 1), (-past, past)):
+        x = _at_level(logn, 0, 4, best[:2], lo, hi)
+        _check_fft(*x, best[3], logn, batch, s, f"largest twiddles, {lo}..{hi}")
+    # and through all windows of such a table, every size of input
+    for amp in (2 ** (np.arange(28, 54) / 2)).astype(int):
+        x = rng.integers(-amp, amp, (2, n), endpoint=True)
+        _check_fft(x[0], x[1], best[3], logn, batch, s, f"largest twiddles, +-{amp}")
     s.destroy()
 
 
