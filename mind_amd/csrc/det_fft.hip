@@ -79,6 +79,8 @@ __host__ __device__ constexpr int32_t i32_bound(int stages, bool peeled) {
     return (int32_t)((2147483647.0 / g - 4.0) / 1.41422);        // > sqrt 2: component -> magnitude
 }
 constexpr int64_t TW_SMALL = 65536;
+// (any int64: no sum that could overflow)
+__device__ __forceinline__ bool in_range(int64_t v, int64_t bound) { return v >= -bound && v <= bound; }
 
 __device__ __forceinline__ uint32_t bitrev(uint32_t v, int bits) { return bits ? __brev(v) >> (32 - bits) : 0u; }
 
@@ -281,8 +283,7 @@ __device__ __forceinline__ bool load_tw32(WinTw &w, const int64_t *__restrict__ 
     bool ok = true;
     each_twiddle<L, NB, P>(low, s, logn, [&](int rb, int q, uint32_t k) {
         const int64_t wr = tw[2 * (size_t)k], wi = tw[2 * (size_t)k + 1];
-        ok = ok && (uint64_t)(wr + TW_SMALL) <= 2 * (uint64_t)TW_SMALL &&
-             (uint64_t)(wi + TW_SMALL) <= 2 * (uint64_t)TW_SMALL;
+        ok = ok && in_range(wr, TW_SMALL) && in_range(wi, TW_SMALL);
         w.r[(1 << rb) - 1 + q] = (int32_t)wr, w.i[(1 << rb) - 1 + q] = (int32_t)wi;
     });
     return ok;
@@ -441,7 +442,7 @@ __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_
         if constexpr (L::FIRST) ok1 = load_tw32<L, NB, 1>(w1, tw, low_bits<L, NB, 1>(t, s, c0), s, logn);
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            ok = ok && (uint64_t)(xr[r] + B) <= 2 * (uint64_t)B && (uint64_t)(xi[r] + B) <= 2 * (uint64_t)B;
+            ok = ok && in_range(xr[r], B) && in_range(xi[r], B);
         if (block_all(ok)) {
             int32_t yr[16], yi[16];
 #pragma unroll
