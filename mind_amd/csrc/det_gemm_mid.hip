@@ -303,12 +303,14 @@ static hipError_t launch(const T *A, const T *B, int32_t *C, int M, int N, int K
 
 // 64 x 64 tiles times 64-k steps: what the kernel's time goes by on full grids.
 static long long mid_tiles(int M, int N) {
-    return (long long)((M + mid::TM - 1) / mid::TM) * ((N + mid::TN - 1) / mid::TN);
+    return ((long long)M + mid::TM - 1) / mid::TM * (((long long)N + mid::TN - 1) / mid::TN);
 }
 static long long mid_work(int M, int N, int K) {
     return mid_tiles(M, N) * ((K + mid::KSTEP - 1) / mid::KSTEP);
 }
-static bool mid_fits(int M, int N) { return N >= mid::TN && mid_tiles(M, N) < (1LL << 28); }
+// A launch holds below 2^32 threads: 2^24 workgroups of 256, rounded up to a
+// multiple of 8 (few rows of 2^30 columns are past that).
+static bool mid_fits(int M, int N) { return N >= mid::TN && mid_tiles(M, N) <= (1LL << 24) - 8; }
 
 // int8, against repacked panels (or the 256 x 256 edge kernel) on shapes that
 // the full-tile kernels do not take as they are; per call, there -> here:

@@ -1920,6 +1920,32 @@ def test_big_gemm_i8():
     np.testing.assert_array_equal(C[rows], O.gemm_i8_rows(A, B, m, k, n, rows))
 
 
+
+def test_big_gemm_i8_past_the_largest_grid():
+    # one row of 2^30 + 77 columns (C = 4 GiB): more 64-column tiles than a
+    # launch holds workgroups of 256 threads
+    m, k, n = 1, 2, (1 << 30) + 77
+    rng = np.random.default_rng(0xB17)
+    A = np.array([-128, 127], np.int8)
+    B = np.resize(rng.integers(-128, 128, (1 << 20) + 7, np.int8), k * n)
+    dA, dB, dC, s = M.DeviceBuffer.from_array(A), M.DeviceBuffer.from_array(B), M.DeviceBuffer(m * n * 4), M.Stream()
+    for how in ("arena", "no_ws"):
+        dC.fill(0xA5)
+        note(f"int8 {m}x{k}x{n} via {how}")
+        if how == "arena":
+            M.check(M.lib().det_matmul_i8_dev(dA.ptr, dB.ptr, dC.ptr, m, k, n, s.ptr))
+        else:
+            M.check(M.lib().det_matmul_ws_dev(M.DET_OP_I8, dA.ptr, dB.ptr, dC.ptr, m, k, n, None, 0, s.ptr))
+        s.sync()
+        got = dC.to_array(np.int32, (n,))
+        for lo in range(0, n, 1 << 27):
+            hi = min(n, lo + (1 << 27))
+            assert np.array_equal(got[lo:hi], -128 * B[lo:hi].astype(np.int32) + 127 * B[n + lo:n + hi].astype(np.int32))
+    s.destroy()
+    for buf in (dA, dB, dC):
+        buf.free()
+
+
 def test_big_gemm_q16_limb_path():
     m, k, n = BIG_M, 16384, 64            # A = 2.5 GiB: beyond the second-generation kernel's limit
     A, B = M.gen_q16(0xB16 ^ 3, m * k, k * n, 13)
