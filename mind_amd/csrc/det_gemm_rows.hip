@@ -201,7 +201,7 @@ bool i8_rows(int M, int N, int K) {
 }
 
 // Workgroups that share a unit's K range: each adds its sums to a zeroed C
-// with integer atomics (so C must be device memory when this is above 1).
+// with integer atomics, which only device memory is sure to take.
 int i8_rows_split(int M, int N, int K) {
     using namespace rows8;
     const int mr = group_rows(M, N), units = (N + TN - 1) / TN * ((M + mr * 16 - 1) / (mr * 16));
@@ -210,9 +210,21 @@ int i8_rows_split(int M, int N, int K) {
     return max(1, min(cus / units, steps / 16));
 }
 
+// Device memory, as opposed to mapped host or managed memory (an atomic there
+// depends on the bus) and to addresses the runtime does not know.
+static bool device_memory(const void *p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();   // handled: clear it
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice;
+}
+
 hipError_t launch_gemm_i8_rows(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s) {
     using namespace rows8;
-    const int split = i8_rows_split(M, N, K);
+    int split = i8_rows_split(M, N, K);
+    if (split > 1 && !device_memory(C)) split = 1;   // plain stores
     switch (group_rows(M, N)) {
     case 1: launch<1, 16, 3>(A, B, C, M, N, K, split, s); break;
     case 2: launch<2, 8, 4>(A, B, C, M, N, K, split, s); break;

@@ -1273,6 +1273,36 @@ def test_gemm_i8_few_rows(m, k, n):
     s.destroy()
 
 
+@pytest.mark.parametrize("m,k,n", [(16, 4096, 1024), (3, 8066, 200)])
+def test_gemm_i8_few_rows_into_host_memory(m, k, n):
+    # C in mapped host memory: no atomic may reach it, though the shape is one
+    # whose K is split over workgroups that add into C
+    split = M.lib()["_ZN3det13i8_rows_splitEiii"]
+    assert split(m, n, k) > 1
+    H = ctypes.CDLL("libamdhip64.so")
+    H.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    H.hipHostFree.argtypes = [ctypes.c_void_p]
+    a, b = O.gen_i8(0x205F ^ k, m * k, k * n)
+    want = O.gemm_i8(a, b, m, k, n)
+    da, db, s, p = M.DeviceBuffer.from_array(a), M.DeviceBuffer.from_array(b), M.Stream(), ctypes.c_void_p()
+    assert H.hipHostMalloc(ctypes.byref(p), m * n * 4, 0) == 0
+    C = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_int32)), (m * n,))
+    for how in ("arena", "no_ws"):
+        C[:] = -1515870811
+        note(f"int8 few rows {m}x{k}x{n}, C in host memory, via {how}")
+        if how == "arena":
+            M.check(M.lib().det_matmul_i8_dev(da.ptr, db.ptr, p.value, m, k, n, s.ptr))
+        else:
+            M.check(M.lib().det_matmul_ws_dev(M.DET_OP_I8, da.ptr, db.ptr, p.value, m, k, n, None, 0, s.ptr))
+        s.sync()
+        np.testing.assert_array_equal(C, want.ravel())
+    del C
+    s.destroy()
+    for buf in (da, db):
+        buf.free()
+    assert H.hipHostFree(p) == 0
+
+
 @pytest.mark.parametrize("m,k,n", RAGGED_I8, ids=[f"{m}x{k}x{n}" for m, k, n in RAGGED_I8])
 @pytest.mark.parametrize("offs", [(0, 0), (1, 3), (8, 4)], ids=["aligned", "off1_3", "off8_4"])
 def test_gemm_i8_ragged_and_misaligned_device_operands(m, k, n, offs):
