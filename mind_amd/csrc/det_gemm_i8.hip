@@ -1507,32 +1507,39 @@ static void launch_i8_on_grid(const int8_t *A, const int8_t *B, int32_t *C, int 
     }
 }
 
+I8Route i8_route(const int8_t *A, const int8_t *B, int M, int N, int K, bool ws) {
+    if (i8_rows(M, N, K)) return I8Route::ROWS;
+    const bool aligned = (((uintptr_t)A & 15) == 0) && (((uintptr_t)B & 15) == 0);
+    const bool small = i8_small(M, N, K);
+    if (small && (K <= I8_SMALL_K || !i8_mid(M, N, K, true))) return I8Route::SMALL;
+    const bool panels = ws && !small && i8_workspace_bytes(M, N, K, aligned) != 0;
+    const bool fast = i8_fast(A, B, M, N, K);
+    if (K >= 1 && !(fast && i8_full_tiles(M, N, K)) && i8_mid(M, N, K, fast || panels)) return I8Route::MID;
+    // A that already suits the full-tile kernels (a ragged or misaligned B,
+    // e.g. N = 4100) stays where it is
+    if (panels) return ((uintptr_t)A & 15) == 0 && M % 128 == 0 && K % 256 == 0 ? I8Route::PANELS_B : I8Route::PANELS;
+    return fast ? I8Route::ON_GRID : I8Route::BYTES;
+}
+
 hipError_t launch_gemm_i8(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, void *ws,
                           hipStream_t s) {
     using namespace i8g;
-    if (i8_rows(M, N, K)) return launch_gemm_i8_rows(A, B, C, M, N, K, s);
-    const bool aligned = (((uintptr_t)A & 15) == 0) && (((uintptr_t)B & 15) == 0);
-    const bool small = i8_small(M, N, K);
-    if (small && (K <= I8_SMALL_K || !i8_mid(M, N, K, true))) return launch_gemm_i8_small(A, B, C, M, N, K, s);
-    const size_t pad = small ? 0 : i8_workspace_bytes(M, N, K, aligned);
-    const bool fast = i8_fast(A, B, M, N, K);
-    if (K >= 1 && !(fast && i8_full_tiles(M, N, K)) && i8_mid(M, N, K, fast || (pad && ws)))
-        return launch_gemm_mid(A, B, C, M, N, K, s);
-    if (fast && !(pad && ws)) {
-        launch_i8_on_grid(A, B, C, M, N, K, N, M, N, s);
-    } else if (pad && ws) {
-        const int Mp = (int)round256(M), Kp = (int)round256(K), Np = (int)round256(N);
-        if (((uintptr_t)A & 15) == 0 && M % 128 == 0 && K % 256 == 0) {
-            // A already suits the full-tile kernels (a ragged or misaligned B,
-            // e.g. N = 1000): repack only B into [K][Np] panels
-            int8_t *Bp = (int8_t *)ws;
-            const int ry = (K + PAD_ROWS - 1) / PAD_ROWS;
-            const dim3 pgrid((unsigned)((Np / 16 + 255) / 256), (unsigned)(ry < 65535 ? ry : 65535), 1);
-            hipLaunchKernelGGL(pad_i8_kernel, pgrid, dim3(256), 0, s, A, B, M, N, K, M, K, Np, (uint4 *)nullptr,
-                               (uint4 *)Bp, 0);
-            launch_i8_on_grid(A, Bp, C, M, Np, K, N, M, N, s);
-            return hipGetLastError();
-        }
+    const int Mp = (int)round256(M), Kp = (int)round256(K), Np = (int)round256(N);
+    switch (i8_route(A, B, M, N, K, ws != nullptr)) {
+    case I8Route::ROWS: return launch_gemm_i8_rows(A, B, C, M, N, K, s);
+    case I8Route::SMALL: return launch_gemm_i8_small(A, B, C, M, N, K, s);
+    case I8Route::MID: return launch_gemm_mid(A, B, C, M, N, K, s);
+    case I8Route::ON_GRID: launch_i8_on_grid(A, B, C, M, N, K, N, M, N, s); break;
+    case I8Route::PANELS_B: {   // B into [K][Np]
+        int8_t *Bp = (int8_t *)ws;
+        const int ry = (K + PAD_ROWS - 1) / PAD_ROWS;
+        const dim3 pgrid((unsigned)((Np / 16 + 255) / 256), (unsigned)(ry < 65535 ? ry : 65535), 1);
+        hipLaunchKernelGGL(pad_i8_kernel, pgrid, dim3(256), 0, s, A, B, M, N, K, M, K, Np, (uint4 *)nullptr,
+                           (uint4 *)Bp, 0);
+        launch_i8_on_grid(A, Bp, C, M, Np, K, N, M, N, s);
+        break;
+    }
+    case I8Route::PANELS: {
         int8_t *Ap = (int8_t *)ws;
         int8_t *Bp = Ap + (size_t)Mp * Kp;
         const int wide = Kp > Np ? Kp : Np, tall = Mp > Kp ? Mp : Kp;
@@ -1541,10 +1548,14 @@ hipError_t launch_gemm_i8(const int8_t *A, const int8_t *B, int32_t *C, int M, i
         hipLaunchKernelGGL(pad_i8_kernel, pgrid, dim3(256), 0, s, A, B, M, N, K, Mp, Kp, Np, (uint4 *)Ap,
                            (uint4 *)Bp, 1);
         launch_i8_on_grid(Ap, Bp, C, Mp, Np, Kp, N, M, N, s);
-    } else {
+        break;
+    }
+    case I8Route::BYTES: {
         const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
         hipLaunchKernelGGL(gemm_i8_kernel<false>, dim3(tiles_m * tiles_n), dim3(THREADS), 0, s, A, B, C, M, N, K,
                            tiles_m, tiles_n);
+        break;
+    }
     }
     return hipGetLastError();
 }

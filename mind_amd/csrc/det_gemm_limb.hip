@@ -372,14 +372,23 @@ size_t i16_workspace_bytes(int M, int N, int K) {
     return a > b ? a : b;
 }
 
+I16Route i16_route(const int16_t *A, const int16_t *B, int M, int N, int K) {
+    const bool on_grid = K % 16 == 0 && N % 8 == 0 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+    const bool small = i16_small(M, N, K);
+    // (up to K = 512 the tiny-shape kernel is as fast: both at the launch floor)
+    if (K >= 1 && i16_mid(M, N, K, on_grid) && !(small && K <= 512)) return I16Route::MID;
+    if (small) return I16Route::SMALL;
+    return i16x_eligible(M, N, K) ? I16Route::INTERLEAVED : I16Route::LIMB;
+}
+
 hipError_t launch_gemm_i16(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K, void *ws,
                            hipStream_t s) {
-    const bool on_grid = K % 16 == 0 && N % 8 == 0 && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
-    const bool use_mid = K >= 1 && i16_mid(M, N, K, on_grid), small = i16_small(M, N, K);
-    // (up to K = 512 the tiny-shape kernel is as fast: both at the launch floor)
-    if (use_mid && !(small && K <= 512)) return launch_gemm_mid(A, B, C, M, N, K, s);
-    if (small) return launch_gemm_i16_small(A, B, C, M, N, K, s);
-    if (i16x_eligible(M, N, K)) return launch_gemm_i16x(A, B, C, M, N, K, ws, s);
+    switch (i16_route(A, B, M, N, K)) {
+    case I16Route::MID: return launch_gemm_mid(A, B, C, M, N, K, s);
+    case I16Route::SMALL: return launch_gemm_i16_small(A, B, C, M, N, K, s);
+    case I16Route::INTERLEAVED: return launch_gemm_i16x(A, B, C, M, N, K, ws, s);
+    case I16Route::LIMB: break;
+    }
     return launch_limb<int16_t, 2, false>(A, B, C, M, N, K, false, ws, s);
 }
 

@@ -22,7 +22,7 @@ constexpr int MAX_CS = 16;
 // on-grid shapes the edge kernel would underfill (i8_edge_underfills),
 // repack the operands into `ws`, which must then hold i8_workspace_bytes(M,
 // N, K, aligned) bytes (0 for every other shape; with ws == NULL they take
-// the byte-load or edge kernel instead).
+// the 64 x 64 tiles, the byte-load or the edge kernel instead: i8_route).
 size_t i8_workspace_bytes(int M, int N, int K, bool aligned);
 // Tiny int8 shapes (det_gemm_small.hip): one direct v_dot4 launch, no
 // workspace, any alignment, when the 16x16 output tiles fit one round of the
@@ -50,6 +50,12 @@ constexpr long long I16_SMALL_K = 4096;
 bool i16_small(int M, int N, int K);
 hipError_t launch_gemm_i16_small(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K,
                                  hipStream_t s);
+// What launch_gemm_i8 does with a call (`ws`: a workspace was given): few
+// rows, tiny shapes, 64 x 64 tiles, full-tile or edge kernels on the operands
+// as they are, the same on panels of B or of both repacked into ws, or the
+// byte-load kernel.
+enum class I8Route { ROWS, SMALL, MID, ON_GRID, PANELS_B, PANELS, BYTES };
+I8Route i8_route(const int8_t *A, const int8_t *B, int M, int N, int K, bool ws);
 hipError_t launch_gemm_i8(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, void *ws,
                           hipStream_t s);
 
@@ -82,6 +88,11 @@ hipError_t launch_gemm_q16(const int32_t *A, const int32_t *B, int32_t *C, int M
 bool q16x_eligible(int M, int N, int K);
 hipError_t launch_gemm_q16x(const int32_t *A, const int32_t *B, int32_t *C, int M, int N, int K, bool b_is_t,
                             void *ws, hipStream_t s);
+// What launch_gemm_i16 does with a call: 64 x 64 tiles, tiny shapes, the
+// interleaved limbs of det_gemm_i16x.hip, or limb planes (operands whose
+// interleave passes 2 GiB).
+enum class I16Route { MID, SMALL, INTERLEAVED, LIMB };
+I16Route i16_route(const int16_t *A, const int16_t *B, int M, int N, int K);
 hipError_t launch_gemm_i16(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K, void *ws,
                            hipStream_t s);
 // int16 as one int8 MFMA GEMM on interleaved limbs (det_gemm_i16x.hip):

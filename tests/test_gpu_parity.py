@@ -15,6 +15,7 @@ import pytest
 
 import mind_amd as M
 import oracle as O
+import routes as R
 
 pytestmark = pytest.mark.gpu
 
@@ -925,7 +926,8 @@ def test_host_batched_gemv_orders_itself_after_device_arena_users():
 # ------------------------------------------------------------------ int8 shapes
 
 # The last three are on the 16-byte grid but off the 128-row kernels with an
-# edge grid under one round: repacked into panels (both operands, or B only).
+# edge grid under one round: a workspace is reported for them, and the 64 x 64
+# tiles take them as they are.  (Shapes for each route: tests/routes.py.)
 I8_SHAPES = [(1, 1, 1), (1, 64, 1), (3, 5, 7), (16, 16, 16), (17, 33, 65), (64, 64, 64), (255, 257, 129),
              (256, 256, 256), (300, 1000, 77), (513, 96, 260), (100, 4096, 8), (8, 4096, 300), (1000, 17, 999),
              (1008, 1008, 1008), (496, 512, 496), (1024, 1024, 1008)]
@@ -944,9 +946,10 @@ def test_gemm_i8_repack_rule_leaves_small_grids_alone():
         assert L.det_workspace_bytes(M.DET_OP_I8, m, k, n) > 0, (m, k, n)
 
 
-# Shapes whose 16x16 output tiles fit one round of the CUs take the direct
-# v_dot4 kernel while K <= 512, or K <= 4096 when M, N or K is not a multiple
-# of 128 (any alignment, no workspace); just past either bound the MFMA
+# Shapes whose 16x16 output tiles fit one round of the CUs need no workspace
+# while K <= 512, or K <= 4096 when M, N or K is not a multiple of 128 (any
+# alignment): the direct v_dot4 kernel, or, with N >= 64, the few-rows kernel
+# (M <= 64) and the 64 x 64 tiles past K = 512; just past either bound other
 # kernels take over (256x640x256, 16x4097x16, 272x16x256: 17 x 16 tiles).
 I8_DIRECT = [(16, 16, 16), (1, 4096, 1), (16, 4096, 16), (256, 512, 256), (255, 4096, 255), (17, 33, 65),
              (5, 1000, 300), (4096, 7, 16), (1, 100, 4096)]
@@ -1128,8 +1131,9 @@ SWEEP_I8 = _sweep_shapes(48, 0x5EE9)
 
 @pytest.mark.parametrize("m,k,n", SWEEP_I8, ids=[f"{m}x{k}x{n}" for m, k, n in SWEEP_I8])
 def test_gemm_i8_routing_sweep(m, k, n):
-    """Every kernel the router can pick, full output against the CPU
-    restatement, through the device entry point (library arena) and through
+    """Shapes over the router's whole range (mostly 64 x 64 and full tiles; one
+    shape or more for every route: test_gpu_routes.py), full output against the
+    CPU restatement, through the device entry point (library arena) and through
     det_matmul_ws_dev with exactly the reported workspace."""
     a, b = O.gen_i8(0x5EE9 ^ (m * 1000003 + k * 1009 + n), m * k, k * n)
     want = _mt_gemm_i8(a, b, m, k, n)
@@ -1172,7 +1176,8 @@ SWEEP_LIMB = [(op, *shape) for op in (M.DET_OP_Q16, M.DET_OP_I16) for shape in _
 @pytest.mark.parametrize("op,m,k,n", SWEEP_LIMB, ids=[f"op{op}-{m}x{k}x{n}" for op, m, k, n in SWEEP_LIMB])
 def test_gemm_limb_sweep(op, m, k, n):
     """Seeded Q16 (saturating generator; direct or limb kernel by shape) and
-    int16 shapes, full output against the CPU restatement, through
+    int16 shapes (64 x 64 tiles or the tiny-shape kernel; limbs:
+    test_gpu_routes.py), full output against the CPU restatement, through
     det_matmul_ws_dev with exactly the reported workspace refilled with
     garbage first."""
     if op == M.DET_OP_Q16:
@@ -1192,11 +1197,12 @@ def test_gemm_limb_sweep(op, m, k, n):
 
 
 # Operands off the 16-byte grid (K or N not a multiple of 16) or not 16-byte
-# aligned: repacked into padded panels in the workspace (arena, caller
-# workspace or scratch), or, without a workspace, the byte-load kernel.
-RAGGED_I8 = [(1, 17, 1),(37, 100, 53), (300, 1000, 77), (256, 4095, 256), (1000, 1000, 1000), (257, 4100, 1003),
+# aligned, with the arena, a workspace or none: kernels that read them where
+# they are at any alignment.  (Larger shapes, which are repacked into padded
+# panels or take the byte-load kernel: test_gpu_routes.py.)
+RAGGED_I8 = [(1, 17, 1), (37, 100, 53), (300, 1000, 77), (256, 4095, 256), (1000, 1000, 1000), (257, 4100, 1003),
              (64, 64, 64), (256, 256, 256),
-             # A on the full-tile grid, B ragged: only B is repacked when A is aligned
+             # A on the full-tile grid, B ragged
              (128, 256, 77), (512, 1024, 1000), (1024, 2048, 1000)]
 
 
@@ -1314,7 +1320,7 @@ def test_gemm_i8_ragged_and_misaligned_device_operands(m, k, n, offs):
     s = M.Stream()
     L = M.lib()
     # the library arena (sized for these addresses), a caller workspace of the
-    # reported size (enough only for aligned operands), and none at all
+    # reported size, and none at all
     ws_bytes = L.det_workspace_bytes(M.DET_OP_I8, m, k, n)
     ws = M.DeviceBuffer(max(ws_bytes, 256))
     for how in ("arena", "ws", "no_ws"):
@@ -1450,14 +1456,6 @@ def test_gemm_q16_multi_tile(gen, shape):
     np.testing.assert_array_equal(c.reshape(m, n), want)
 
 
-# Shapes whose 16x16 tiles times K are too much for the direct kernel run
-# the limb kernel; its grids of 64 x 64 tiles that fill at most half the CUs
-# run split in K (up to 8 partial sums per tile over whole 64-k steps,
-# reduced by a second kernel): 7 x 5000 x 130 (3 tiles, K off the 64 grid,
-# splits of 9-10 steps), 100 x 4200 x 70 (4 ragged tiles, uneven splits),
-# 200 x 4160 x 300 (20 tiles), 1000 x 4100 x 33 (16 tiles, one column), 512 x
-# 2048 x 512 (64 tiles, 4 splits of 8 steps); 1000 x 100 x 1000 and 1024 x
-# 128 x 1024 fill the chip (no split; the first ragged in M, N and K).
 # Direct-kernel shapes beyond those that report no workspace (5 to 10 rounds of
 # 16 x 16 tiles), each just inside and just past the rule's limits: the same
 # integers on either route.
@@ -1472,6 +1470,14 @@ def test_gemm_q16_direct_rounds(m, k, n):
     np.testing.assert_array_equal(M.det_matmul_q16(a.reshape(m, k), b.reshape(k, n)), O.gemm_q16(a, b, m, k, n))
 
 
+# Shapes whose 16x16 tiles times K are too much for the direct kernel run
+# the limb kernel; its grids of 64 x 64 tiles that fill at most half the CUs
+# run split in K (up to 8 partial sums per tile over whole 64-k steps,
+# reduced by a second kernel): 7 x 5000 x 130 (3 tiles, K off the 64 grid,
+# splits of 9-10 steps), 100 x 4200 x 70 (4 ragged tiles, uneven splits),
+# 200 x 4160 x 300 (20 tiles), 1000 x 4100 x 33 (16 tiles, one column), 512 x
+# 2048 x 512 (64 tiles, 4 splits of 8 steps); 1000 x 100 x 1000 and 1024 x
+# 128 x 1024 fill the chip (no split; the first ragged in M, N and K).
 Q_SPLIT = [(7, 5000, 130), (100, 4200, 70), (200, 4160, 300), (1000, 4100, 33), (512, 2048, 512), (1000, 100, 1000),
            (1024, 128, 1024)]
 
@@ -1479,15 +1485,15 @@ Q_SPLIT = [(7, 5000, 130), (100, 4200, 70), (200, 4160, 300), (1000, 4100, 33), 
 @pytest.mark.parametrize("m,k,n", Q_SPLIT, ids=[f"{m}x{k}x{n}" for m, k, n in Q_SPLIT])
 def test_gemm_q16_k_split(m, k, n):
     """The limb route (split in K where the grid is small) against the
-    oracle: saturating inputs through the
-    device workspace entry (the workspace, partials included, refilled with
-    garbage before each call), and full-range inputs through gemmqmm and the
+    oracle: saturating inputs through the device workspace entry (the
+    workspace, partials included, refilled with garbage before each call), and
+    full-range inputs through gemmqmm and the
     B-transposed gemmq."""
     L = M.lib()
     a, b = O.gen_q16_sat(0x5A17 ^ (m * 7919 + k * 31 + n), m * k, k * n, shift=13)
     want = O.gemm_q16(a, b, m, k, n).reshape(m, n)
     wsb = L.det_workspace_bytes(M.DET_OP_Q16, m, k, n)
-    assert wsb > 0   # the limb route (the direct kernel needs no workspace)
+    assert wsb > 0 and not R.q16_direct(m, k, n)   # the limb route
     s = M.Stream()
     da, db, dc = M.DeviceBuffer.from_array(a), M.DeviceBuffer.from_array(b), M.DeviceBuffer(m * n * 4)
     ws = M.DeviceBuffer(wsb)
@@ -1513,9 +1519,10 @@ def test_gemm_q16_k_split(m, k, n):
     np.testing.assert_array_equal(c, want.ravel())
 
 
-# int16 shapes whose 16x16 output tiles fit one round of the CUs take the
-# direct v_dot2 kernel while K <= 4096 (no workspace); just past either
-# bound (16x4097x16, 272x16x256) the limb-interleaved MFMA GEMM takes over.
+# int16 shapes whose 16x16 output tiles fit one round of the CUs need no
+# workspace while K <= 4096: the direct v_dot2 kernel, or, with N >= 64 and
+# past K = 512, the 64 x 64 tiles; just past either bound the interleaved limbs
+# (16x4097x16) or the tiles (272x16x256) take over.
 I16_DIRECT = [(16, 16, 16), (1, 4096, 1), (16, 4096, 16), (255, 4096, 255), (17, 33, 65), (256, 256, 256),
               (4096, 9, 16), (1, 100, 4096)]
 I16_DIRECT_EDGE = [(16, 4097, 16), (272, 16, 256)]
@@ -1592,9 +1599,9 @@ GEMV_FULL = [(64, 512, 2), (300, 1024, 3), (130, 2048, 8), (16, 32768, 8)]
 @pytest.mark.parametrize("fam", ["full", "extreme"])
 @pytest.mark.parametrize("m,k,nb", GEMV_FULL, ids=[f"{m}x{k}b{nb}" for m, k, nb in GEMV_FULL])
 def test_gemv_q16_batched_full_range(m, k, nb, fam):
-    """The batched (MFMA) path on full-range int32 W and x: every limb of W and
-    every digit of x in use (x near 2^31 - 1 needs the fifth digit), up to the
-    kernel's largest K."""
+    """Batched calls on full-range int32 W and x: every limb of W and every
+    digit of x in use.  (These have too few rows for the MFMA kernel:
+    test_gpu_routes.py has the same inputs at shapes that take it.)"""
     rng = np.random.default_rng(m * 31 + k + nb + len(fam))
     ext = np.array([2147483647, -2147483648, -2147483647, 2139062144, 2139062143, 0, 1, -1, 65535, -65536,
                     -8421505, 8421504], np.int32)
@@ -1613,9 +1620,10 @@ GEMV_WS = [(64, 512, 8), (1000, 1024, 13), (16, 32768, 2), (300, 512, 1), (130, 
 @pytest.mark.parametrize("m,k,nb", GEMV_WS, ids=[f"{m}x{k}b{nb}" for m, k, nb in GEMV_WS])
 def test_gemv_q16_ws_dev(m, k, nb):
     """det_gemv_q16_ws_dev: the caller's workspace (garbage-filled, exactly
-    det_gemv_workspace_bytes), a workspace one byte short and none at all
-    (both take the one-vector kernel) give the oracle's output, twice in a
-    row on poisoned outputs; 130 x 1000 (K % 512 != 0) needs no workspace."""
+    det_gemv_workspace_bytes), a workspace one byte short and none at all give
+    the oracle's output, twice in a row on poisoned outputs; 130 x 1000 (K % 512
+    != 0) needs no workspace.  (All on the VALU kernel, with too few rows for
+    the MFMA kernel; test_gpu_routes.py compares the two.)"""
     L = M.lib()
     W, X = O.gen_q16(0x6E5 ^ (m * k + nb), m * k, nb * k, shift=0)
     want = O.gemv_q16_batched(W, X, m, k, nb).reshape(nb, m)
@@ -1751,6 +1759,7 @@ def test_ws_dev_exact_workspace_with_garbage(op, m, k, n):
     # the exact reported workspace, refilled with garbage before every call:
     # the preps write every column-sum partial they later read (several
     # 64-row B tiles per partial at these K), nothing relies on zeroed memory
+    # (int16 here runs on tiles that use none; with limbs: test_gpu_routes.py)
     if op == "i16":
         a, b = O.gen_i16(0x6A5 ^ k, m * k, k * n)
         want, code, dt = O.gemm_i16(a, b, m, k, n), M.DET_OP_I16, np.int16
@@ -1949,6 +1958,15 @@ def test_big_gemm_i8():
     rows = np.unique(np.r_[_sample_rows(m, 12), (1 << 31) // k - 1, (1 << 31) // k])
     np.testing.assert_array_equal(C[rows], O.gemm_i8_rows(A, B, m, k, n, rows))
 
+
+def test_big_gemm_i8_mid_tiles():
+    m, k, n = 65536, 40960, 72            # A = 2.5 GiB on the 64 x 64 tiles: no panels of that size
+    assert R.i8(m, k, n) == R.i8(m, k, n, 1, 3) == "mid"
+    A, B = M.gen_i8(0xB16 ^ 8, m * k, k * n)
+    note(f"det_matmul_i8_dev {m}x{k}x{n} (A {A.nbytes >> 20} MiB)")
+    C = _dev_run(lambda pa, pb, pc, s: M.lib().det_matmul_i8_dev(pa, pb, pc, m, k, n, s), [A, B], (m, n), reps=1)
+    rows = np.unique(np.r_[_sample_rows(m, 12), (1 << 31) // k - 1, (1 << 31) // k])
+    np.testing.assert_array_equal(C[rows], O.gemm_i8_rows(A, B, m, k, n, rows))
 
 
 def test_big_gemm_i8_past_the_largest_grid():

@@ -5,8 +5,9 @@ grid in a third of the cases) and through the host-pointer det_matmul_*
 calls; the Q16 GEMV at batch 1..9, the int16 GEMV, the Q16 / L1 / int16
 dots and the strict-FP f32 rows at random lengths; the Q16 FFT at random
 sizes and batches.  Shapes mix tiny, odd, near-power-of-two and mid-size
-dimensions so that the router's every branch is drawn (tiny direct
-kernels, MFMA kernels, repack, K split, limb kernels).  GEMM rows are
+dimensions so that most of the router's branches are drawn (tiny direct
+kernels, 64 x 64 tiles, K split, limb kernels; all of them:
+test_gpu_routes.py).  GEMM rows are
 sampled (first, last and three random ones); everything else is checked
 whole."""
 import numpy as np

@@ -2,9 +2,10 @@
 det_matmul_ws_dev (the existing workspace entry point) through the C ABI:
 bit-identical outputs on two calls in a row, the second smaller, for the
 int16 and Q16 limb GEMMs (which use the scratch; the Q16 shapes here are too
-large for the direct kernel, which needs none) and int8 (which uses it only
-to repack operands into padded panels); a limb-GEMM shape beyond the fixed
-scratch is rejected before any launch.  The property the entry
+large for the direct kernel, which needs none; small int16 ones run on the
+64 x 64 tiles, which need none either) and int8 (which uses it only to repack
+operands into padded panels); a limb-GEMM shape beyond the fixed scratch is
+rejected before any launch.  The property the entry
 point exists for is checked directly: after one warm-up call per op, further
 calls leave the device's free memory unchanged, and one call per op captured
 into a HIP graph (capture fails on hipMalloc or any synchronising call)
@@ -17,6 +18,7 @@ import pytest
 
 import mind_amd as M
 import oracle as O
+import routes as R
 
 pytestmark = pytest.mark.gpu
 
@@ -77,8 +79,9 @@ def test_scratch_entry_matches_workspace_entry_twice(op):
 
 def test_scratch_entry_int8_repack_twice():
     # both shapes are off the 16-byte grid (K % 16 != 0) and too large for
-    # the direct kernel: their padded panels come from the scratch, the
-    # second call's smaller ones over the first's
+    # the direct kernel: panels are reported for them, the second call's
+    # smaller than the first's (the 64 x 64 tiles take both and leave the
+    # scratch alone: test_scratch_entry_panels_and_limbs_twice)
     L, f = _bind()
     s = M.Stream()
     for shape in ((1000, 1000, 77), (700, 200, 90)):
@@ -86,6 +89,26 @@ def test_scratch_entry_int8_repack_twice():
     assert L.det_workspace_bytes(M.DET_OP_I8, 1000, 1000, 77) > L.det_workspace_bytes(M.DET_OP_I8, 700, 200, 90)
     _run_both(L, f, M.DET_OP_I8, 1000, 1000, 77, 0x5C5, s)
     _run_both(L, f, M.DET_OP_I8, 700, 200, 90, 0x5C6, s)
+    s.destroy()
+
+
+# padded panels of both operands, of B alone, int16 limbs: the second call's,
+# smaller, go over the first one's
+SCRATCH = {"panels": ((M.DET_OP_I8, 2500, 1001, 1500), (M.DET_OP_I8, 2111, 650, 1999)),
+           "panels_b": ((M.DET_OP_I8, 2048, 1024, 2000), (M.DET_OP_I8, 2048, 768, 2060)),
+           "interleaved": ((M.DET_OP_I16, 1000, 5000, 1200), (M.DET_OP_I16, 1100, 4001, 900))}
+
+
+@pytest.mark.parametrize("route", sorted(SCRATCH))
+def test_scratch_entry_panels_and_limbs_twice(route):
+    L, f = _bind()
+    s = M.Stream()
+    large, small = SCRATCH[route]
+    for op, *shape in (large, small):
+        assert (R.i8 if op == M.DET_OP_I8 else R.i16)(*shape) == route
+    assert 32 << 20 >= L.det_workspace_bytes(*large) > L.det_workspace_bytes(*small) > 0
+    _run_both(L, f, *large, 0x5C7, s)
+    _run_both(L, f, *small, 0x5C8, s)
     s.destroy()
 
 
@@ -158,8 +181,8 @@ def test_scratch_entry_allocates_nothing_and_captures_into_a_graph():
     H = _hip()
     s = M.Stream()
     # one shape per op within the scratch (Q16: one on the limb kernel split
-    # in K, one on the direct kernel, which uses no scratch); the int8 one off
-    # the 16-byte grid, so its panels come from the scratch
+    # in K, one on the direct kernel, which uses no scratch; int16 and int8 run
+    # on the 64 x 64 tiles, which use none: the routes that do are below)
     cases = [(M.DET_OP_Q16, 200, 4160, 300, 0x5D1), (M.DET_OP_Q16, 256, 512, 192, 0x5D4),
              (M.DET_OP_I16, 320, 1088, 272, 0x5D2), (M.DET_OP_I8, 1000, 1000, 77, 0x5D3)]
     bufs = []
@@ -208,5 +231,60 @@ def test_scratch_entry_allocates_nothing_and_captures_into_a_graph():
         H.hipGraphDestroy(graph)
     for op, m, k, n, da, db, c_eager, c_graph, want in bufs:
         for buf in (da, db, c_eager, c_graph):
+            buf.free()
+    s.destroy()
+
+
+def test_scratch_entry_panels_limbs_and_few_rows_in_a_graph():
+    """The routes that write to the scratch, and int8 with few rows and K split,
+    which asks the runtime what C is: no allocation, and captured as above."""
+    L, f = _bind()
+    H = _hip()
+    s = M.Stream()
+    cases = [SCRATCH["interleaved"][1], SCRATCH["panels"][1], SCRATCH["panels_b"][1], (M.DET_OP_I8, 16, 4096, 1024)]
+    assert [(R.i8 if op == M.DET_OP_I8 else R.i16)(*shape) for op, *shape in cases] == \
+        ["interleaved", "panels", "panels_b", "rows"]
+    bufs = []
+    for i, (op, m, k, n) in enumerate(cases):
+        a, b, want = _inputs(op, m, k, n, 0x5D5 + i)
+        print(f"[no-alloc graph] op={op} {m}x{k}x{n}", flush=True)
+        bufs.append((op, m, k, n, M.DeviceBuffer.from_array(a), M.DeviceBuffer.from_array(b),
+                     M.DeviceBuffer(m * n * 4), want.reshape(m, n)))
+
+    def calls():
+        return [f(op, da.ptr, db.ptr, c.ptr, m, k, n, s.ptr) for op, m, k, n, da, db, c, want in bufs]
+
+    def check():
+        for op, m, k, n, da, db, c, want in bufs:
+            np.testing.assert_array_equal(c.to_array(np.int32, (m, n)), want)
+            c.fill(0x5A)
+
+    assert calls() == [0] * len(bufs)
+    s.sync()
+    free0 = _free_bytes(H)
+    for _ in range(3):
+        assert calls() == [0] * len(bufs)
+        s.sync()
+    assert _free_bytes(H) == free0
+    check()
+    graph, exe = ctypes.c_void_p(0), ctypes.c_void_p(0)
+    assert H.hipStreamBeginCapture(s.ptr, 1) == 0
+    rcs = calls()
+    assert H.hipStreamEndCapture(s.ptr, ctypes.byref(graph)) == 0
+    assert rcs == [0] * len(bufs), (rcs, M.last_error())
+    assert H.hipGraphInstantiateWithFlags(ctypes.byref(exe), graph, 0) == 0
+    try:
+        for replay in range(3):
+            assert H.hipGraphLaunch(exe, s.ptr) == 0
+            s.sync()
+            check()
+            assert calls() == [0] * len(bufs)   # eager work on the same scratch between replays
+            s.sync()
+            check()
+    finally:
+        H.hipGraphExecDestroy(exe)
+        H.hipGraphDestroy(graph)
+    for op, m, k, n, da, db, c, want in bufs:
+        for buf in (da, db, c):
             buf.free()
     s.destroy()
