@@ -161,21 +161,21 @@ __global__ __launch_bounds__(256) void fft_small_kernel(const int64_t *__restric
 // the short transforms in one kernel with an all-or-nothing int32 test that
 // left n >= 1024 in int64; one global-memory pass per 4 stages beyond, whose
 // first pass gathered single 8-byte points):
-//   65536 x 256 points 102.7 -> 94 us (5.7 TB/s; a large copy reaches 5.2),
-//   32768 x 512 150 -> 100, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 116,
-//   100000 x 64 80 -> 38, 100000 x 128 102 -> 68, 300000 x 32 335 -> 55;
-//   up to 4% slower where the launch is most of the time (513 x 64 6.1 -> 6.3),
-//   and 9000 - 12000 x 128 9.5 - 11.0 -> 10.3 - 11.3;
+//   65536 x 256 points 102 -> 95 us (5.6 TB/s; a large copy reaches 5.2),
+//   32768 x 512 146 -> 102, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 120,
+//   100000 x 64 87 -> 38, 100000 x 128 104 -> 68, 300000 x 32 355 -> 55,
+//   8192 x 128 10.0 -> 8.9, 5000 x 128 8.2 -> 8.0, 1000 x 256 7.35 -> 7.4;
 //   16 x 2^16 points 86.1 -> 25.5 (34 MB read and written once: 6.6 us at the
 //   copy rate; the two passes wait for memory, then compute, with one workgroup
 //   per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
 //   61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7.
-// Inputs within 2^40 (int64): 65536 x 256 114 -> 117, 32768 x 512 190 -> 134,
-//   13594 x 1024 231 -> 136, 8192 x 2048 302 -> 173, 100000 x 64 73 -> 50,
-//   100000 x 128 104 -> 96, 12000 x 128 13.8 -> 14.5, 16 x 2^16 86 -> 36.
+// Inputs within 2^40 (int64): 65536 x 256 113 -> 116, 8192 x 256 15.9 -> 16.3,
+//   32768 x 512 191 -> 133, 13594 x 1024 231 -> 137, 8192 x 2048 301 -> 172,
+//   100000 x 64 81 -> 50, 100000 x 128 105 -> 95, 6144 x 128 10.7 -> 10.9, 16 x
+//   2^16 86 -> 36.
 // Inputs up to 2^25, where a later window's test fails (before: int64
-// throughout; restarting; going on): 65536 x 256 114, 162, 109 us, 8192 x 256
-// 16.3, 20.0, 14.5, 600 x 512 12.5, 14.8, 10.9, 300 x 1024 10.8, 12.2, 9.5,
+// throughout; restarting; going on): 65536 x 256 113, 162, 110 us, 8192 x 256
+// 16.1, 20.7, 14.7, 600 x 512 12.5, 14.8, 10.9, 300 x 1024 10.8, 12.2, 9.5,
 // 16 x 2048 11.6, 13.2, 10.2 (2^22: 11.6, 15.0, 9.0).
 // Window P of NB bits: first bit of its 4 registers, and the stages it runs.
 template <int NB, int P>
@@ -485,18 +485,15 @@ __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_
 
 // 4096 consecutive points per workgroup: 16 transforms of 256 points and so
 // on.  Points past the batch load as zero and are not stored.  Staging adds
-// two LDS exchanges to save partial-line requests: always at 32 points (8000
-// transforms 7.0 us against 10.5 without; 2000 6.8 against 8.1), at 64 from
-// 2^18 points (8000: 7.4 against 9.7), at 128 from 5 x 2^18 (16000: 12.4
-// against 14.8; 8192: 9.0 against 9.1, but inputs past 2^26, read again in the
-// other order, 12.1 against 10.7); a 256-point transform's 16 lanes cover whole
-// lines as they are.
-constexpr int64_t stage_points(int logn) { return logn == 5 ? 0 : logn == 6 ? 1 << 18 : 5 << 18; }
-
-template <int LOGN, bool STAGED>
+// two LDS exchanges to save partial-line requests: below 256 points, whose 16
+// lanes cover whole lines as they are (8000 x 32 points 7.0 us against 10.5
+// without, 8000 x 64 7.4 against 9.7; 5000 x 128 8.0 against 8.8, 16000 12.5
+// against 16.1; inputs past 2^26, read again in the other order, 5000 10.4
+// against 10.2, 16000 17.0 against 19.9).
+template <int LOGN>
 __global__ __launch_bounds__(256) void fft_rows_kernel(const int64_t *sre, const int64_t *sim, int64_t *dre,
                                                        int64_t *dim, const int64_t *__restrict__ tw, int64_t points) {
-    using L = RowsLay<LOGN, STAGED>;
+    using L = RowsLay<LOGN, (LOGN < 8)>;
     constexpr int NP = (LOGN + 3) / 4;
     __shared__ uint64_t sm[L::ELEMS];
     const int64_t off = (int64_t)blockIdx.x << 12;
@@ -591,19 +588,28 @@ static void launch_cols(const int64_t *sre, const int64_t *sim, int64_t *dre, in
 // barrier-separated stages instead of a lane walking its 16 points through
 // every stage.  Same butterflies, same stage order: same bits.  Loads and
 // stores touch each point once (an in-place call reads all of its transform
-// before writing, at the first barrier).  Per call, this against the window
-// kernels (with about 7 us of host submission in both): 256 points x16 7.2
-// against 7.2 us (inputs up to 2^40: 7.2 against 9.0), 512 points x128 7.2
-// against 8.3, 1024 points x128 7.5 against 7.2 (7.5 against 9.1), but x512
-// 11.4 against 8.1, and 2048 points x1 11.3 against 7.7, x512 21.0 against
-// 14.9.
-constexpr int few_batch(int logn) { return logn <= 9 ? 512 : logn == 10 ? 256 : 0; }
+// before writing, at the first barrier).  LDS is sized by n: at 24 KiB for every
+// n six workgroups fit a compute unit (4096 x 32 points 8.3 us, now 5.0; 3000 x
+// 128 8.3, now 6.2).
+// Device time per call, this against the window kernels, inputs within 2^16
+// (2^40): 256 points x100 4.2 against 6.9 us (9.2), x768 5.6 against 7.2 (9.4),
+// x1536 7.7 against 7.5 (9.8); 32 x8192 7.1 against 7.3 (9.3), x12288 9.2
+// against 7.5; 64 x6144 7.2 against 7.7 (10.0), x8192 8.6 against 8.1; 128 x4096
+// 7.4 against 7.6 (9.4), x6144 9.9 against 8.7; 512 x512 7.1 against 8.7 (10.8),
+// x1024 10.4 against 9.2; 1024 x256 7.7 against 6.6 (9.6), x300 10.6 against
+// 7.2 (10.8).
+constexpr int few_batch(int logn) {
+    constexpr int most[] = {8192, 6144, 4096, 768, 512, 256};
+    return logn >= 5 && logn <= 10 ? most[logn - 5] : 0;
+}
 
-__global__ __launch_bounds__(512) void fft_few_kernel(const int64_t *__restrict__ sre, const int64_t *__restrict__ sim,
-                                                       int64_t *dre, int64_t *dim, const int64_t *__restrict__ tw,
-                                                       int logn) {
-    __shared__ int64_t lre[1024], lim[1024], ltw[1024];
-    const int n = 1 << logn, half_n = n >> 1, t = threadIdx.x;
+template <int LOGN>
+__global__ __launch_bounds__((1 << LOGN) / 2) void fft_few_kernel(const int64_t *__restrict__ sre,
+                                                                  const int64_t *__restrict__ sim, int64_t *dre,
+                                                                  int64_t *dim, const int64_t *__restrict__ tw) {
+    constexpr int logn = LOGN, n = 1 << logn, half_n = n >> 1;
+    __shared__ int64_t lre[n], lim[n], ltw[n];
+    const int t = threadIdx.x;
     const size_t base = (size_t)blockIdx.x * n;
     for (int i = t; i < n; i += blockDim.x) {   // bit reversal on the way in
         const uint32_t p = bitrev((uint32_t)i, logn);
@@ -691,8 +697,8 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
 #define LDS(LG)                                                                                                \
     case LG: {                                                                                                 \
         if (batch <= few_batch(LG)) {                                                                          \
-            hipLaunchKernelGGL(fft_few_kernel, dim3((unsigned)batch), dim3((1u << LG) / 2), 0, s, sre, sim, dre, dim, \
-                               tw, LG);                                                                        \
+            hipLaunchKernelGGL(fft_few_kernel<(LG < 10 ? LG : 10)>, dim3((unsigned)batch), dim3((1u << LG) / 2), 0, s, \
+                               sre, sim, dre, dim, tw);                                                        \
             break;                                                                                             \
         }                                                                                                      \
         if constexpr (LG >= 10) {                                                                              \
@@ -701,12 +707,7 @@ hipError_t launch_fft_q16(const int64_t *sre, const int64_t *sim, int64_t *dre, 
         } else {                                                                                               \
             const int64_t points = batch << LG;                                                                \
             const dim3 grid((unsigned)((points + 4095) / 4096));                                               \
-            if (LG < 8 && points >= stage_points(LG))                                                          \
-                hipLaunchKernelGGL((fft_rows_kernel<LG, (LG < 8)>), grid, dim3(256), 0, s, sre, sim, dre, dim, tw, \
-                                   points);                                                                    \
-            else                                                                                               \
-                hipLaunchKernelGGL((fft_rows_kernel<LG, false>), grid, dim3(256), 0, s, sre, sim, dre, dim, tw, \
-                                   points);                                                                    \
+            hipLaunchKernelGGL(fft_rows_kernel<LG>, grid, dim3(256), 0, s, sre, sim, dre, dim, tw, points);    \
         }                                                                                                      \
         break;                                                                                                 \
     }

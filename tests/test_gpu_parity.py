@@ -530,16 +530,17 @@ def test_fft_out_of_place_and_path_choice():
         b.free()
 
 
-# More than 512 transforms of 32 to 2048 points (the batched kernels, each with
-# a partly filled last workgroup; linear staging at 64 points from 2^18 points
-# and at 128 from 5 x 2^18), and of 4096 points and more: whole transforms per
-# workgroup (4096 points; 8192 from a batch of 128) or column passes of 6 to 9 stages (every
-# width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
+# Transforms of 32 to 2048 points: a few (a workgroup each: up to 8192, 6144,
+# 4096, 768, 512 and 256 of 32 to 1024 points) and more (the batched kernels,
+# each with a partly filled last workgroup); and of 4096 points and more: whole
+# transforms per workgroup (4096 points; 8192 from a batch of 128) or column
+# passes of 6 to 9 stages (every width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
 # scratch) and out of place.  Amplitudes: Q16; about 44.7 million, which passes
 # the first window's test and fails a later one's (the block then goes on in
 # int64, or starts again); +-2^40.
 FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (7, 10243), (8, 513), (9, 515), (10, 256), (10, 257),
               (11, 513), (12, 2), (13, 127), (13, 128), (14, 3), (15, 2), (16, 1), (17, 1), (18, 1), (19, 1)]
+FFT_PASSES += [(5, 8192), (5, 8193), (6, 6144), (6, 6147), (7, 4096), (7, 4097), (8, 768), (8, 769), (9, 512)]
 
 
 @pytest.mark.parametrize("logn,batch", FFT_PASSES, ids=[f"n{1 << l}_b{b}" for l, b in FFT_PASSES])
@@ -643,9 +644,10 @@ def _check_fft(re, im, tw, logn, batch, s, what):
         b.free()
 
 
-# (logn, batch, stages of each pass): short transforms, staged and not; a
+# (logn, batch, stages of each pass): short transforms in batches past a few,
+# staged (up to 128 points) and not; a
 # transform per workgroup; column passes
-FFT_BOUNDS = [(5, 600, [5]), (6, 600, [6]), (6, 4100, [6]), (7, 600, [7]), (7, 10300, [7]), (8, 600, [8]),
+FFT_BOUNDS = [(5, 8200, [5]), (6, 6200, [6]), (7, 4100, [7]), (7, 10300, [7]), (8, 770, [8]),
               (9, 600, [9]), (10, 300, [10]), (11, 3, [11]), (12, 2, [12]), (13, 128, [13]), (13, 2, [7, 6]),
               (15, 1, [8, 7]), (17, 1, [9, 8])]
 
