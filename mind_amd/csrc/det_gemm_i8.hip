@@ -1511,10 +1511,10 @@ I8Route i8_route(const int8_t *A, const int8_t *B, int M, int N, int K, bool ws)
     if (i8_rows(M, N, K)) return I8Route::ROWS;
     const bool aligned = (((uintptr_t)A & 15) == 0) && (((uintptr_t)B & 15) == 0);
     const bool small = i8_small(M, N, K);
-    if (small && (K <= I8_SMALL_K || !i8_mid(M, N, K, true))) return I8Route::SMALL;
-    const bool panels = ws && !small && i8_workspace_bytes(M, N, K, aligned) != 0;
     const bool fast = i8_fast(A, B, M, N, K);
-    if (K >= 1 && !(fast && i8_full_tiles(M, N, K)) && i8_mid(M, N, K, fast || panels)) return I8Route::MID;
+    if (small && (K <= I8_SMALL_K || !i8_mid(M, N, K, true, fast))) return I8Route::SMALL;
+    const bool panels = ws && !small && i8_workspace_bytes(M, N, K, aligned) != 0;
+    if (K >= 1 && !(fast && i8_full_tiles(M, N, K)) && i8_mid(M, N, K, fast || panels, fast)) return I8Route::MID;
     // A that already suits the full-tile kernels (a ragged or misaligned B,
     // e.g. N = 4100) stays where it is
     if (panels) return ((uintptr_t)A & 15) == 0 && M % 128 == 0 && K % 256 == 0 ? I8Route::PANELS_B : I8Route::PANELS;

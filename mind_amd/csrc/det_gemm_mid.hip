@@ -312,30 +312,68 @@ static long long mid_work(int M, int N, int K) {
 // multiple of 8 (few rows of 2^30 columns are past that).
 static bool mid_fits(int M, int N) { return N >= mid::TN && mid_tiles(M, N) <= (1LL << 24) - 8; }
 
-// int8, against repacked panels (or the 256 x 256 edge kernel) on shapes that
-// the full-tile kernels do not take as they are; per call, there -> here:
+// int8, against repacked panels (or the 256 x 256 edge kernel, on the 16-byte
+// grid) on shapes that the full-tile kernels do not take as they are; device
+// time per call, there -> here:
 //   up to one tile per compute unit: 384 x 2735 x 338 21.1 -> 14.2 us,
 //     1024 x 1920 x 822 (208 tiles) 16.4 -> 9.3, 1001^3 12.6 -> 8.1, 1500 x
 //     4000 x 500 25.8 -> 18.2, 463 x 256 x 1792 11.2 -> 7.4;
-//   beyond: 1300^3 (9261 tile steps) 15.8 -> 13.9, 2000 x 256 x 2000 12.0 -> 7.2,
-//     3000 x 300 x 3000 (11045) 26.1 -> 23.0, but 2000 x 700 x 2000 (11264)
-//     15.1 -> 16.4 and 2000^3 20 -> 30: 64 x 64 tiles read each operand from L2
-//     four times as often as 256 x 256 ones.
+//   beyond: 1300^3 (9261 tile steps) 17.8 -> 13.4, 2000 x 300 x 2000 13.5 -> 11.8,
+//     3000 x 300 x 3000 (11045) 26.6 -> 23.5.
+// Past that, 256 x 256 tiles there read each operand from L2 a fourth as often,
+// so a step costs them less.  With a K remainder, a step of its own in every round
+// of tiles here, the crossover therefore lies at fewer steps the more rounds there
+// are (a last one here, a first one there):
+//   on the grid, against one round of 256 x 256 tiles: 4 rounds 2000 x 624 x 2000
+//     (10 steps) 15.8 -> 15.4, 2000 x 752 14.6 -> 17.4; 5 rounds 3008 x 240 x 1408
+//     12.4 -> 11.9, 15008 x 368 x 304 13.4 -> 15.6; 6 rounds 2304 x 112 x 2304 11.3 ->
+//     9.8, 2304 x 304 13.1 -> 15.8; 9 rounds 3008 x 48 x 3008 11.1 -> 10.2, 3008 x
+//     176 13.1 -> 17.6; but against two rounds 3392 x 96 x 4704 21.9 -> 17.9;
+//   off it, against one round of little padded 128 x 128 tiles: 3 rounds 2609 x 559
+//     x 1009 14 -> 13, 1505 x 687 x 1505 13 -> 14; 4 rounds 2001 x 303 x 2001 14 ->
+//     13, 2001 x 495 13.5 -> 15.5; of 128 x 256 tiles: 5 rounds 977 x 367 x 5009 17
+//     -> 16, 3009 x 431 x 1409 17 -> 18; 7 rounds 2513 x 111 x 2513 18 -> 12, 2513 x
+//     367 18 -> 21.  Rows on the 4-byte grid load faster here: 1500 x 900 x 1500 14.2
+//     -> 13.2, 2000 x 500 x 2000 13.5 -> 13.1, but 2000 x 600 14.2 -> 15.0; 3159 x 521
+//     x 1376 (5 rounds) 19.4 -> 15.4, 2677 x 257 x 2352 (7) 18.0 -> 15.4, but 2500 x
+//     380 x 2500 18.4 -> 20.3.
+// Of 700 drawn shapes near these lines the taken kernel is the slower one by more
+// than 4% for 30, by 14% at most where it is this one, 25% where not.
+// Without a remainder all of these stay faster here: 2000 x 640 x 2000 16.0 -> 11.5,
+//   4688 x 576 x 896 15.2 -> 11.7, 3008 x 192 x 3008 13 -> 10, 2513 x 512 x 2512 18 ->
+//   17, 4000 x 192 x 4000 16 -> 16.
 // Without a workspace the alternative for operands off the 16-byte grid is the
 // byte-load kernel (4095^3 829 us; here 280): any size.
-bool i8_mid(int M, int N, int K, bool panels) {
+bool i8_mid(int M, int N, int K, bool panels, bool on_grid) {
     if (!mid_fits(M, N)) return false;
     if (!panels) return true;
-    return (mid_tiles(M, N) <= cu_count() && K <= 8192) || mid_work(M, N, K) <= 11100;
+    const long long cus = cu_count(), tiles = mid_tiles(M, N), rounds = (tiles + cus - 1) / cus;
+    const long long steps = ((long long)K + mid::KSTEP - 1) / mid::KSTEP;
+    if (rounds == 1 && K <= 8192) return true;
+    if (tiles * steps > 11100) return false;
+    if (rounds <= 2 || K % mid::KSTEP == 0) return true;
+    const long long m256 = ((long long)M + 255) / 256, n256 = ((long long)N + 255) / 256;
+    if (on_grid) return m256 * n256 > cus || rounds <= 4 || steps <= (rounds == 5 ? 4 : rounds <= 7 ? 2 : 1);
+    const bool one_round = m256 * n256 * 2 <= cus;   // of 128 x 256 tiles
+    const bool little_padded = min(M, N) >= 512 && 4 * 65536 * m256 * n256 <= 5LL * M * N;
+    if (!one_round || !little_padded) return true;
+    if (m256 * n256 * 4 <= cus)   // 128 x 128 tiles
+        return K % 4 == 0 && N % 4 == 0 ? rounds == 3 || rounds * steps <= 34 : rounds * steps <= 27;
+    return rounds * steps <= (N % 4 ? (rounds <= 4 ? 40 : 30) : rounds <= 5 ? 50 : 36);
 }
 
 // int16, against the operand prep plus the interleaved limb GEMM, whose prep
 // reads by element off the 16-byte grid:
 //   up to one tile per compute unit: 1024^3 17.9 -> 10.6, 1403 x 791 x 640
 //     21.1 -> 11.7, 300 x 2000 x 300 36.2 -> 18.6, 1024 x 2048 x 1024 26.5 -> 17.5;
-//   beyond, off the grid: 1200^3 26.7 -> 20.4, 1500^3 (13824 tile steps) 34.8 ->
-//     34.0; on it: 2000 x 300 x 2000 (5120; K off) 20.0 -> 17.4, but 2048^3
-//     (32768) 39 -> 58.
+//   beyond, off the grid: 1200^3 27.9 -> 20.3, 1500^3 (13824 tile steps) 37.4 ->
+//     32.7, 3009 x 527 x 1409 39 -> 33, 3009 x 367 x 3009 47 -> 41, 4001 x 175 x 4001
+//     48 -> 44; on it: 1280^3 (8000) 25.0 -> 18.9, 2048 x 512 x 2048 19.8 -> 17.7,
+//     2304 x 176 x 2304 22 -> 17, but 2048^3 (32768) 39 -> 58.
+// The crossover in tile steps varies from family to family, so the limits lie
+// where nearly all are faster here: on 1300^2 and 800 x 1700 it is past 30000, but
+// at 2000^2, where the limbs fill exactly one round of 256 x 256 tiles, 10000 off
+// the grid (2000 x 601 x 2000 24.0 -> 25.4, the largest loss) and 7500 on it.
 bool i16_mid(int M, int N, int K, bool on_grid) {
     if (!mid_fits(M, N)) return false;
     return (mid_tiles(M, N) <= cu_count() && K <= 4096) || mid_work(M, N, K) <= (on_grid ? 8000 : 14000);

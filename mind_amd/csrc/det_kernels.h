@@ -39,9 +39,9 @@ hipError_t launch_gemm_i8_rows(const int8_t *A, const int8_t *B, int32_t *C, int
 // int8 / int16 GEMM in one launch on 64 x 64 tiles (det_gemm_mid.hip): no
 // workspace, any alignment, N >= 64.  i8_mid: for shapes the full-tile kernels
 // do not take as they are, `panels` if the alternative is repacked panels or
-// the edge kernel; i16_mid: `on_grid` if the alternative's prep reads whole
-// 16-byte vectors.
-bool i8_mid(int M, int N, int K, bool panels);
+// the edge kernel, `on_grid` if operands and sizes are on the 16-byte grid;
+// i16_mid: `on_grid` if the alternative's prep reads whole 16-byte vectors.
+bool i8_mid(int M, int N, int K, bool panels, bool on_grid);
 bool i16_mid(int M, int N, int K, bool on_grid);
 hipError_t launch_gemm_mid(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
 hipError_t launch_gemm_mid(const int16_t *A, const int16_t *B, int32_t *C, int M, int N, int K, hipStream_t s);

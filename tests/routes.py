@@ -37,8 +37,8 @@ def i8_workspace(m, k, n, aligned):
     return rule("_ZN3det18i8_workspace_bytesEiiib", m, n, k, aligned, restype=ctypes.c_size_t)
 
 
-def i8_mid(m, k, n, panels=False):
-    return rule("_ZN3det6i8_midEiiib", m, n, k, panels)
+def i8_mid(m, k, n, panels=False, on_grid=False):
+    return rule("_ZN3det6i8_midEiiibb", m, n, k, panels, on_grid)
 
 
 def q16_direct(m, k, n):
@@ -70,7 +70,17 @@ I8_ROUTES = [
     # byte loads: off the grid, fewer than 64 columns, no workspace
     (5000, 300, 50, (0, 0), False, "bytes"), (4100, 1037, 63, (1, 3), False, "bytes"),
     (70000, 3, 17, (0, 0), False, "bytes"), (65, 5000, 33, (0, 0), False, "bytes"),
-    # 64 x 64 tiles without a workspace: any size off the grid
+    # 64 x 64 tiles against one round of larger tiles: few steps and rounds; on
+    # the grid; rows on the 4-byte grid; much padding; several rounds there
+    (2001, 350, 2001, (0, 0), True, "mid"), (2001, 490, 2001, (0, 0), True, "panels"),
+    (2304, 112, 2304, (0, 0), True, "mid"), (2304, 304, 2304, (0, 0), True, "on_grid"),
+    (3008, 112, 3008, (0, 0), True, "on_grid"), (3008, 48, 3008, (0, 0), True, "mid"),
+    (2000, 500, 2000, (0, 0), True, "mid"), (2000, 600, 2000, (0, 0), True, "panels"),
+    (209, 431, 16001, (0, 0), True, "mid"), (3009, 250, 3009, (0, 0), True, "mid"),
+    (3159, 521, 1376, (0, 0), True, "mid"), (2513, 367, 2513, (0, 0), True, "panels"),
+    # (no K remainder; two rounds of tiles here)
+    (2512, 384, 2512, (0, 0), True, "mid"), (1869, 1673, 676, (0, 0), True, "mid"),
+    # and without a workspace: any size off the grid
     (2111, 650, 1999, (0, 0), False, "mid"), (2048, 768, 2064, (1, 3), False, "mid"),
 ]
 # int16 as interleaved limbs: off the grid (by size, by address), on it, few rows

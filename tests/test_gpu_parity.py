@@ -534,8 +534,8 @@ def test_fft_out_of_place_and_path_choice():
 # 4096, 768, 512 and 256 of 32 to 1024 points) and more (the batched kernels,
 # each with a partly filled last workgroup); and of 4096 points and more: whole
 # transforms per workgroup (4096 points; 8192 from a batch of 128) or column
-# passes of 6 to 9 stages (every width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 = 7 + 6 + 6), in place (through
-# scratch) and out of place.  Amplitudes: Q16; about 44.7 million, which passes
+# passes of 6 to 9 stages (every width: 13 = 7 + 6, 15 = 8 + 7, 17 = 9 + 8, 19 =
+# 7 + 6 + 6), in place (through scratch) and out of place.  Amplitudes: Q16; about 44.7 million, which passes
 # the first window's test and fails a later one's (the block then goes on in
 # int64, or starts again); +-2^40.
 FFT_PASSES = [(5, 513), (6, 519), (6, 4099), (7, 515), (7, 8195), (7, 10243), (8, 513), (9, 515), (10, 256), (10, 257),
