@@ -200,8 +200,8 @@ bool i8_rows(int M, int N, int K) {
            !(K <= I8_SMALL_K && i8_small(M, N, K));
 }
 
-// Workgroups that share a unit's K range: each adds its sums to a zeroed C
-// with integer atomics, which only device memory is sure to take.
+// Workgroups that share a unit's K range: each adds its sums to a zeroed C with
+// integer atomics, which only this device's memory is sure to take.
 int i8_rows_split(int M, int N, int K) {
     using namespace rows8;
     const int mr = group_rows(M, N), units = (N + TN - 1) / TN * ((M + mr * 16 - 1) / (mr * 16));
@@ -210,15 +210,17 @@ int i8_rows_split(int M, int N, int K) {
     return max(1, min(cus / units, steps / 16));
 }
 
-// Device memory, as opposed to mapped host or managed memory (an atomic there
-// depends on the bus) and to addresses the runtime does not know.
+// Memory of the current device, as opposed to mapped host or managed memory or
+// another device's (an atomic there depends on the bus) and to addresses the
+// runtime does not know.
 static bool device_memory(const void *p) {
     hipPointerAttribute_t at;
-    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    int d = -1;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || hipGetDevice(&d) != hipSuccess) {
         (void)hipGetLastError();   // handled: clear it
         return false;
     }
-    return at.type == hipMemoryTypeDevice;
+    return at.type == hipMemoryTypeDevice && at.device == d;
 }
 
 hipError_t launch_gemm_i8_rows(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s) {
