@@ -500,8 +500,9 @@ int64_t gemm_host(Op op, int64_t a, int64_t b, int64_t c, int64_t m, int64_t k, 
     if ((rc = ensure(&ds.ws, &ds.ws_bytes, need))) return rc;
     const bool pinned = pinned_route(ds, span);
     hipStream_t s = ds.stream;
-    // the tiny-shape kernels over at most 16 output tiles read the inputs
-    // from the pinned buffer itself when the layout is small
+    // shapes of at most 16 output tiles of 16 x 16 (tiny-shape kernels, or few
+    // rows and 64 x 64 tiles where those are taken) read the inputs from the
+    // pinned buffer itself when the layout is small
     const int M = (int)m, N = (int)n, K = (int)k;
     const bool tiny = op == Op::I8 ? det::i8_small(M, N, K) : op == Op::I16 ? det::i16_small(M, N, K)
                                                                             : det::q16_small(M, N, K);
@@ -924,7 +925,8 @@ int64_t det_matmul_ws_dev(int64_t op, const void *a, const void *b, int32_t *c, 
     const size_t need = ws_need(o, m, k, n, a, b);
     const bool enough = ws_bytes >= 0 && (size_t)ws_bytes >= need && (need == 0 || ws);
     // int8 runs without a workspace too (operands off the 16-byte grid then
-    // take the byte-load kernel); the limb GEMMs cannot
+    // take the 64 x 64 tiles, or the byte-load kernel below 64 columns); the
+    // limb GEMMs cannot
     if (!enough && o != Op::I8) return set_err(DET_ERR_ARG, "workspace too small (see det_workspace_bytes)");
     return gemm_dev(o, a, b, c, m, k, n, enough ? ws : nullptr, (hipStream_t)stream);
 }

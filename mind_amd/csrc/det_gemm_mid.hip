@@ -337,8 +337,8 @@ static bool mid_fits(int M, int N) { return N >= mid::TN && mid_tiles(M, N) <= (
 //     -> 13.2, 2000 x 500 x 2000 13.5 -> 13.1, but 2000 x 600 14.2 -> 15.0; 3159 x 521
 //     x 1376 (5 rounds) 19.4 -> 15.4, 2677 x 257 x 2352 (7) 18.0 -> 15.4, but 2500 x
 //     380 x 2500 18.4 -> 20.3.
-// Of 700 drawn shapes near these lines the taken kernel is the slower one by more
-// than 4% for 30, by 14% at most where it is this one, 25% where not.
+// Of 230 drawn shapes near these lines the taken kernel is the slower one by more
+// than 4% for 7, by 14% at most where it is this one, 25% where not.
 // Without a remainder all of these stay faster here: 2000 x 640 x 2000 16.0 -> 11.5,
 //   4688 x 576 x 896 15.2 -> 11.7, 3008 x 192 x 3008 13 -> 10, 2513 x 512 x 2512 18 ->
 //   17, 4000 x 192 x 4000 16 -> 16.

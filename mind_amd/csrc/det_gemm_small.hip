@@ -115,7 +115,8 @@ static long long small_tiles(int M, int N) {
 // K > 512 on shapes their full 128-row tiles take (128x1024x128: 5.3 against
 // 6.4 us).  Other shapes would go to the edge or byte-load kernels or be
 // repacked first, which costs more up to K = 4096 (16x4096x16: 38 against
-// 20 us; 300x1000x77: 13.3 against 7.5 us).
+// 20 us); from 64 columns on and past K = 512 the few-rows kernel or the 64 x
+// 64 tiles take them instead (i8_route).
 bool i8_small(int M, int N, int K) {
     if (K < 1 || small_tiles(M, N) > cu_count()) return false;
     const bool mfma_tiles = M % 128 == 0 && N % 128 == 0 && K % 128 == 0;

@@ -27,7 +27,8 @@ size_t i8_workspace_bytes(int M, int N, int K, bool aligned);
 // Tiny int8 shapes (det_gemm_small.hip): one direct v_dot4 launch, no
 // workspace, any alignment, when the 16x16 output tiles fit one round of the
 // compute units and K <= I8_SMALL_K, or K <= I8_SMALL_K_ODD for shapes the
-// full-tile MFMA kernels do not take (M, N or K not a multiple of 128).
+// full-tile MFMA kernels do not take (M, N or K not a multiple of 128; past
+// I8_SMALL_K those of 64 columns or more go to the two kernels below).
 constexpr long long I8_SMALL_K = 512, I8_SMALL_K_ODD = 4096;
 bool i8_small(int M, int N, int K);
 hipError_t launch_gemm_i8_small(const int8_t *A, const int8_t *B, int32_t *C, int M, int N, int K, hipStream_t s);
