@@ -162,20 +162,20 @@ __global__ __launch_bounds__(256) void fft_small_kernel(const int64_t *__restric
 // left n >= 1024 in int64; one global-memory pass per 4 stages beyond, whose
 // first pass gathered single 8-byte points):
 //   65536 x 256 points 102 -> 95 us (5.6 TB/s; a large copy reaches 5.2),
-//   32768 x 512 146 -> 102, 13594 x 1024 231 -> 89, 8192 x 2048 302 -> 120,
-//   100000 x 64 87 -> 38, 100000 x 128 104 -> 68, 300000 x 32 355 -> 55,
-//   8192 x 128 10.0 -> 8.9, 5000 x 128 8.2 -> 8.0, 1000 x 256 7.35 -> 7.4;
+//   32768 x 512 146 -> 99, 13594 x 1024 231 -> 90, 8192 x 2048 302 -> 115,
+//   100000 x 64 87 -> 34, 100000 x 128 104 -> 66, 300000 x 32 355 -> 48,
+//   8192 x 128 10.0 -> 9.2, 5000 x 128 8.2 -> 8.3, 1000 x 256 7.5 -> 7.5;
 //   16 x 2^16 points 86.1 -> 25.5 (34 MB read and written once: 6.6 us at the
 //   copy rate; the two passes wait for memory, then compute, with one workgroup
 //   per compute unit), 32 x 2^16 128 -> 36.4, 8 x 2^18 148 -> 44.2, 1 x 2^16
 //   61 -> 17.1, 512 x 4096 91 -> 20.6, 256 x 8192 94 -> 25.7.
-// Inputs within 2^40 (int64): 65536 x 256 113 -> 116, 8192 x 256 15.9 -> 16.3,
-//   32768 x 512 191 -> 133, 13594 x 1024 231 -> 137, 8192 x 2048 301 -> 172,
-//   100000 x 64 81 -> 50, 100000 x 128 105 -> 95, 6144 x 128 10.7 -> 10.9, 16 x
+// Inputs within 2^40 (int64): 65536 x 256 113 -> 115, 8192 x 256 16.3 -> 16.3,
+//   32768 x 512 191 -> 136, 13594 x 1024 231 -> 135, 8192 x 2048 301 -> 172,
+//   100000 x 64 81 -> 46, 100000 x 128 105 -> 87, 5000 x 128 10.3 -> 10.2, 16 x
 //   2^16 86 -> 36.
 // Inputs up to 2^25, where a later window's test fails (before: int64
-// throughout; restarting; going on): 65536 x 256 113, 162, 110 us, 8192 x 256
-// 16.1, 20.7, 14.7, 600 x 512 12.5, 14.8, 10.9, 300 x 1024 10.8, 12.2, 9.5,
+// throughout; restarting; going on): 65536 x 256 113, 161, 108 us, 8192 x 256
+// 16.3, 20.6, 14.9, 600 x 512 12.5, 14.8, 10.9, 300 x 1024 10.8, 12.2, 9.5,
 // 16 x 2048 11.6, 13.2, 10.2 (2^22: 11.6, 15.0, 9.0).
 // Window P of NB bits: first bit of its 4 registers, and the stages it runs.
 template <int NB, int P>
@@ -214,9 +214,10 @@ struct RowsLay {   // 4096 consecutive points: 2^(12 - NB) whole short transform
     // STAGED: loads and stores are linear and go through LDS (below 256 points
     // a window's lanes cover less than a 128-byte line of each transform).
     // The int64 path, 16 bytes a point, is staged below 128 points only.
-    // KEEP: inputs that fail window 0's test stay in registers (same layout;
-    // 600 x 32 points in +-2^40 9.9 us read again, 8.7 kept).
-    static constexpr bool STAGED = STAGED_, KEEP = !STAGED || NB < 7, RESUME = true;
+    // KEEP: inputs that fail window 0's test stay in registers.  Staged ones are
+    // read again, which leaves a third wave per SIMD (300000 x 32 points 54 us
+    // kept, 48 read again, 100000 x 64 38, 34; in +-2^40 65, 62 and 49, 46).
+    static constexpr bool STAGED = STAGED_, KEEP = !STAGED, RESUME = true;
     using Wide = RowsLay<NB, STAGED_ && (NB < 7)>;
     template <int P>
     static __device__ __forceinline__ uint32_t label(uint32_t t) {
@@ -354,14 +355,28 @@ __device__ __forceinline__ void exchange(T (&x)[16], uint32_t t, T *sm) {
     __syncthreads();
 }
 
+// The same for int32 pairs, in two halves: to LDS as window P - 1 has them, and
+// back (widened if V is int64_t) as window P wants them.
+template <class L, int NB, int P>
+__device__ __forceinline__ void put32(const int32_t (&yr)[16], const int32_t (&yi)[16], uint32_t t, uint64_t *sm) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        sm[elem<L, NB, P - 1>(t, r)] = (uint64_t)(uint32_t)yr[r] | ((uint64_t)(uint32_t)yi[r] << 32);
+    __syncthreads();
+}
+template <class L, int NB, int P, typename V>
+__device__ __forceinline__ void get32(V (&yr)[16], V (&yi)[16], uint32_t t, const uint64_t *sm) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const uint64_t z = sm[elem<L, NB, P>(t, r)];
+        yr[r] = (int32_t)(uint32_t)z, yi[r] = (int32_t)(uint32_t)(z >> 32);
+    }
+    __syncthreads();
+}
 template <class L, int NB, int P>
 __device__ __forceinline__ void exchange32(int32_t (&yr)[16], int32_t (&yi)[16], uint32_t t, uint64_t *sm) {
-    uint64_t z[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) z[r] = (uint64_t)(uint32_t)yr[r] | ((uint64_t)(uint32_t)yi[r] << 32);
-    exchange<L, NB, P>(z, t, sm);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) yr[r] = (int32_t)(uint32_t)z[r], yi[r] = (int32_t)(uint32_t)(z[r] >> 32);
+    put32<L, NB, P>(yr, yi, t, sm);
+    get32<L, NB, P>(yr, yi, t, sm);
 }
 
 template <class L, int NB, int P>
@@ -374,8 +389,8 @@ __device__ __forceinline__ uint32_t low_bits(uint32_t t, int s, uint32_t c0) {
 // (L::FIRST) w holds window P's (w_ok: all small), loaded one window ahead;
 // in later passes that would cost the second wave per SIMD (16 transforms of
 // 2^16 25.8 us instead of 27, 32 of them 41.9 instead of 38.6), so they are
-// loaded here.  Returns the window whose test failed (the values are then its
-// inputs), or NP when all have run.
+// loaded here.  Returns the window whose test failed (L::RESUME: its inputs
+// are then in LDS), or NP when all have run.
 template <class L, int NB, int P>
 __device__ __forceinline__ int narrow_from(int32_t (&yr)[16], int32_t (&yi)[16], const int64_t *__restrict__ tw,
                                            uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, WinTw &w, bool w_ok) {
@@ -394,32 +409,36 @@ __device__ __forceinline__ int narrow_from(int32_t (&yr)[16], int32_t (&yi)[16],
         }
         const bool fits = block_all(w_ok && hi <= B && lo >= -B);
         if (!L::RESUME && !fits) return P;
-        exchange32<L, NB, P>(yr, yi, t, sm);
+        put32<L, NB, P>(yr, yi, t, sm);
         if (!fits) return P;
+        get32<L, NB, P>(yr, yi, t, sm);
         run_win32<L, NB, P>(yr, yi, w);
         return narrow_from<L, NB, P + 1>(yr, yi, tw, t, s, c0, logn, sm, wn, wn_ok);
     }
     return P;
 }
 
-// Windows P.. of the int64 path, or those from `from` on (uniform, at least P),
-// whose inputs x then holds.
 template <class L, int NB, int P>
+__device__ __forceinline__ void exchange64(int64_t (&xr)[16], int64_t (&xi)[16], uint32_t t, uint64_t *sm) {
+    exchange<L, NB, P>(xr, t, (int64_t *)sm);
+    exchange<L, NB, P>(xi, t, (int64_t *)sm);
+}
+
+// Windows P.. of the int64 path, or those from `from` on (uniform): x holds
+// window P's inputs if P >= from, later inputs are where the int32 path left them
+// in LDS.  (W's labels are L's from window 1 on.)
+template <class L, class W, int NB, int P>
 __device__ __forceinline__ void wide_from(int64_t (&xr)[16], int64_t (&xi)[16], const int64_t *__restrict__ tw,
                                           uint32_t t, int s, uint32_t c0, int logn, uint64_t *sm, int from) {
     constexpr int NP = (NB + 3) / 4;
     if constexpr (P < NP) {
-        if (NP == 2 || from <= P) {
-            if ((P > 0 || L::STAGED) && from < P) {
-                exchange<L, NB, P>(xr, t, (int64_t *)sm);
-                exchange<L, NB, P>(xi, t, (int64_t *)sm);
-            }
-            run_win64<L, NB, P>(xr, xi, tw, low_bits<L, NB, P>(t, s, c0), s, logn);
+        if (from <= P) {
+            run_win64<W, NB, P>(xr, xi, tw, low_bits<W, NB, P>(t, s, c0), s, logn);
+            if constexpr (P + 1 < NP || W::STAGED) exchange64<W, NB, P + 1>(xr, xi, t, sm);
+        } else if (P + 1 < NP && from == P + 1) {
+            get32<L, NB, P + 1>(xr, xi, t, sm);
         }
-        wide_from<L, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm, from);
-    } else if constexpr (L::STAGED) {
-        exchange<L, NB, P>(xr, t, (int64_t *)sm);
-        exchange<L, NB, P>(xi, t, (int64_t *)sm);
+        wide_from<L, W, NB, P + 1>(xr, xi, tw, t, s, c0, logn, sm, from);
     }
 }
 
@@ -456,29 +475,35 @@ __device__ __forceinline__ void run_pass(const int64_t *__restrict__ tw, uint32_
                 for (int r = 0; r < 16; ++r) store(L(), t, r, (int64_t)yr[r], (int64_t)yi[r]);
                 return;
             }
-            if constexpr (L::RESUME)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) xr[r] = yr[r], xi[r] = yi[r];
         }
     }
     using W = typename L::Wide;
+    // One copy of each int64 window, entered with inputs from LDS: values held
+    // across the branch cost 128 points the third wave per SIMD (100000 in +-2^40
+    // 87 -> 95 us).
     if constexpr (L::RESUME) {
         // LDS positions and addresses of its own: sharing the int32 path's
         // would hold them in registers across it
         asm volatile("" : "+v"(t));
-        if (from) {   // W's labels are L's from window 1 on
-            wide_from<W, NB, 1>(xr, xi, tw, t, s, c0, logn, sm, from);
+    } else {
+        from = 0;   // again from the source
+    }
+    if (from == 0) {
+        if (!L::KEEP) {
+            // the twiddles of a test that failed have come: or each load would
+            // wait for the one before (100000 x 128 in +-2^40 87 -> 128 us)
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+            asm volatile("" ::: "memory");
 #pragma unroll
-            for (int r = 0; r < 16; ++r) store(W(), t, r, xr[r], xi[r]);
-            return;
+            for (int r = 0; r < 16; ++r) load(W(), t, r, xr[r], xi[r]);
         }
+        if constexpr (W::STAGED) exchange64<W, NB, 0>(xr, xi, t, sm);
+        run_win64<W, NB, 0>(xr, xi, tw, low_bits<W, NB, 0>(t, s, c0), s, logn);
+        exchange64<W, NB, 1>(xr, xi, t, sm);
+    } else if (from == 1) {
+        get32<L, NB, 1>(xr, xi, t, sm);
     }
-    if (!L::KEEP) {
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int r = 0; r < 16; ++r) load(W(), t, r, xr[r], xi[r]);
-    }
-    wide_from<W, NB, 0>(xr, xi, tw, t, s, c0, logn, sm, -1);
+    wide_from<L, W, NB, 1>(xr, xi, tw, t, s, c0, logn, sm, from);
 #pragma unroll
     for (int r = 0; r < 16; ++r) store(W(), t, r, xr[r], xi[r]);
 }
