@@ -371,9 +371,11 @@ bool i8_mid(int M, int N, int K, bool panels, bool on_grid) {
 //     48 -> 44; on it: 1280^3 (8000) 25.0 -> 18.9, 2048 x 512 x 2048 19.8 -> 17.7,
 //     2304 x 176 x 2304 22 -> 17, but 2048^3 (32768) 39 -> 58.
 // The crossover in tile steps varies from family to family, so the limits lie
-// where nearly all are faster here: on 1300^2 and 800 x 1700 it is past 30000, but
-// at 2000^2, where the limbs fill exactly one round of 256 x 256 tiles, 10000 off
-// the grid (2000 x 601 x 2000 24.0 -> 25.4, the largest loss) and 7500 on it.
+// where no family loses much: at 2000^2, where the limbs fill exactly one round of
+// 256 x 256 tiles, it is 10000 off the grid (2000 x 601 x 2000 24.0 -> 25.4, the
+// largest loss) and 7500 on it; on 1300^2 and 800 x 1700 it is past 30000, and
+// 1550^3 (15625) and 1700^3 (19683), past the limit, would gain as well (41.0 -> 33.4,
+// 43.6 -> 37.8).
 bool i16_mid(int M, int N, int K, bool on_grid) {
     if (!mid_fits(M, N)) return false;
     return (mid_tiles(M, N) <= cu_count() && K <= 4096) || mid_work(M, N, K) <= (on_grid ? 8000 : 14000);
