@@ -5,10 +5,11 @@
 // (the batched form of __mind_blas_gemv_q16_mt: reference src/mlir/lowering.rs:
 // 9822-9997; oracle benches/det_gemv_q16_mt.rs:186-197).
 //
-// Why: the one-vector kernel (det_gemv.hip) spends ~8 VALU slots per term on
-// the 64-bit product; with 8 vectors that is ~4x the VALU budget HBM speed
-// allows.  Here, per W element, the VALU only splits W into limbs and
-// computes the residue for each vector (1 op per term):
+// Why: the VALU kernel (det_gemv.hip) spends 20 issue cycles per wave and term,
+// with 8 vectors 1.7 times what the stream of W allows (8192^2 71 us of issue
+// against 41).  Here, per W element, the VALU only splits W into limbs and
+// computes the residue for each vector (1 op per term); gemv8_pays() says which
+// groups of vectors that is the faster way for:
 //   * S = sum_k W x exactly (mod 2^48) from int8 limb-pair MFMAs.  W is
 //     written as signed int8 limbs t_p (low bytes biased by -128 = u ^ 0x80,
 //     c = 0x808080): W = sum_p 2^(8p) t_p + c.  The query vectors (small,
